@@ -60,6 +60,38 @@ def test_block_pre_and_post_match_oracle(cuda, tokens):
     assert torch.equal(res, out)
 
 
+@pytest.mark.parametrize("tokens,hidden,experts,inter", [
+    (11, 256, 63, 64),     # the smallest tiled call; the shared gate fills the router tile's last row
+    (64, 136, 64, 40),     # one full row tile; the shared gate alone in a tile; K and inter past a step / tile
+    (65, 1032, 13, 104),   # one row in the second row tile
+    (130, 264, 5, 8),      # the smallest inter
+])
+def test_block_tiled_calls_match_oracle(cuda, tokens, hidden, experts, inter):
+    """Tile edges of the many-token kernels, with padded row strides."""
+    print_case("moe block tiled", tokens, hidden, experts, inter)
+    g = torch.Generator().manual_seed(tokens)
+    rw, sw, gw, uw, dw = weights(hidden, experts, inter, g)
+
+    def padded(t):
+        wide = torch.full((t.shape[0], t.shape[1] + 8), float("nan"), dtype=t.dtype, device=cuda)
+        wide[:, :t.shape[1]] = t.to(cuda)
+        return wide[:, :t.shape[1]]
+
+    x, after, experts_out = (torch.randn(tokens, hidden, generator=g).bfloat16() for _ in range(3))
+    blk = block.MoeBlock(padded(rw), sw.to(cuda), padded(gw), padded(uw), padded(dw), None, None, top_k=4)
+    logits, sgate, act = blk.pre(padded(x))
+    want_logits, want_sgate, want_act = orc.block_pre(as_np(x), as_np(rw), as_np(sw), as_np(gw), as_np(uw))
+    assert np.max(np.abs(as_np(logits) - want_logits)) <= 2 * BF16_STEP * np.max(np.abs(want_logits))
+    assert np.max(np.abs(as_np(sgate) - want_sgate)) <= 2 * BF16_STEP
+    assert np.max(np.abs(as_np(act) - want_act)) <= 2 * BF16_STEP * np.max(np.abs(want_act))
+    out = blk.post(act, sgate, padded(experts_out), padded(after))
+    want = orc.block_post(as_np(act), as_np(dw), as_np(sgate), as_np(experts_out), as_np(after))
+    assert rel_inf(as_np(out), want) < 1e-2
+    # the same rows one by one through the GEMV: bf16 roundings of sums in another order
+    one = torch.cat([blk.pre(x[t:t + 1].to(cuda))[0] for t in range(tokens)])
+    assert np.max(np.abs(as_np(one) - as_np(logits))) <= BF16_STEP * np.max(np.abs(want_logits))
+
+
 @pytest.mark.parametrize("tokens", [1, 4])
 def test_moe_block_full_shape_fp8(cuda, tokens):
     """Hidden 2048, 128 FP8 experts of 768 (per-channel scales), top-8, a
