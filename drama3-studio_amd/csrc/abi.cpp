@@ -385,9 +385,10 @@ void fp8_decode_call(const BankGeom& g, Activations a, const dmoe::RouteSource& 
 // workspace serves both paths.
 using dmoe::PrefillWorkspace;
 
-size_t prefill_workspace_layout(int pairs, int experts, int H, int I, void* base, PrefillWorkspace* ws) {
+size_t prefill_workspace_layout(int pairs, int experts, int H, int I, void* base, PrefillWorkspace* ws,
+                                bool h32 = false) {
     dmoe::Carver c(base);
-    const PrefillWorkspace w = dmoe::prefill_layout(c, pairs, experts, H, I);
+    const PrefillWorkspace w = dmoe::prefill_layout(c, pairs, experts, H, I, h32);
     if (ws) *ws = w;
     return c.size();
 }
@@ -556,18 +557,33 @@ void check_quant_rows(const void* x, int x_dtype, int64_t x_row_stride, int rows
     require(row_div >= 1 && (int64_t)(pairs - 1) / row_div < rows, "pairs read past the activation rows");
 }
 
-// A grouped packed projection: the tiled W4A16 GEMM where its tile shape
-// fits, else the column-group kernel.
-void launch_projection(const dmoe::QuantProjArgs& q, int max_active, int pairs, hipStream_t stream) {
-    if (dmoe::w4a16_grouped_fits(q)) dmoe::launch_w4a16_grouped(q, max_active, stream, pairs);
-    else dmoe::launch_quant_projection(q, max_active, stream);
+// A grouped packed projection: the tiled 8-bit GEMM (modes 1-3), the tiled
+// W4A16 GEMM where its tile shape fits, else the column-group kernel.
+void launch_projection(const dmoe::QuantProjArgs& q, const QuantWorkspace& ws, int experts, int pairs,
+                       hipStream_t stream) {
+    const int max_active = std::min(pairs, experts);
+    if (dmoe::packed_grouped_fits(q.mode, q.N, q.K, q.w_sn, q.s_sn)) {
+        dmoe::PackedGroupedArgs a{};
+        a.p = q;
+        a.tile_expert = ws.tile_expert;
+        a.tile_m0 = ws.tile_m0;
+        a.tile_count = ws.tile_count;
+        a.max_tiles = std::min(pairs, dmoe::max_block_tiles(pairs, experts, dmoe::kGroupM));
+        dmoe::launch_packed_grouped(a, stream);
+    } else if (dmoe::w4a16_grouped_fits(q)) {
+        dmoe::launch_w4a16_grouped(q, max_active, stream, pairs);
+    } else {
+        dmoe::launch_quant_projection(q, max_active, stream);
+    }
 }
 
 // Permutation with the active-expert list (the grouping of every packed call).
 void quant_group(const void* ids, int ids_dtype, int pairs, int experts, const QuantWorkspace& ws, int* status,
                  hipStream_t stream) {
     dmoe::PermuteArgs pa{ids, ids_dtype, pairs, experts, ws.order, ws.counts, ws.offsets, status,
-                         ws.permute_scratch, ws.permute_scratch + pairs, ws.active, 0, 0, nullptr, nullptr};
+                         ws.permute_scratch, ws.permute_scratch + pairs, ws.active, dmoe::kGroupM,
+                         dmoe::max_block_tiles(pairs, experts, dmoe::kGroupM), ws.tile_expert, ws.tile_m0,
+                         ws.tile_count};
     dmoe::launch_permute(pa, stream);
 }
 
@@ -637,13 +653,94 @@ BankGeom check_g128_bank(const DmoeQuantBank* bank) {
 
 size_t element_size(int dtype) { return dtype == DMOE_F32 || dtype == DMOE_I32 ? 4 : dtype == DMOE_I64 ? 8 : 2; }
 
-// A group-128 call of any size from route ids as consecutive decode calls of
-// at most kMaxDecodePairs pairs, in order on the stream (pairs of a chunk
-// read rows of their own; layer outputs are cut at whole tokens).
+// A large group-128 call as tiled grouped GEMMs: activation quantization (with
+// `ra` the router in the same launch), permutation + tile map, gate/up, hidden
+// quantization, down, combine.
+void g128_grouped_call(const BankGeom& g, const Activations& x, const dmoe::RouteArgs* ra, const void* ids,
+                       int ids_dtype, const void* weights, int weights_dtype, int pairs, int top_k, void* out,
+                       int out_dtype, int64_t out_row_stride, float* out_pairs, void* workspace, int* status,
+                       hipStream_t stream) {
+    PrefillWorkspace ws{};
+    prefill_workspace_layout(pairs, g.experts, g.H, g.I, workspace, &ws, true);
+    const int rows = (pairs - 1) / x.row_div + 1, tiles = dmoe::max_block_tiles(pairs, g.experts, dmoe::kGroupM);
+    const dmoe::QuantArgs qa{x.x, x.x_dtype, x.x_row_stride, rows, g.H, g.H, 0, ws.xq, ws.xs, status, 1};
+    if (ra) dmoe::launch_route_quantize(*ra, qa, stream);
+    else dmoe::launch_fp8_quantize(qa, stream);
+    const dmoe::PermuteArgs pa{ids, ids_dtype, pairs, g.experts, ws.order, ws.counts, ws.offsets, status,
+                               ws.permute_scratch, ws.permute_scratch + pairs, nullptr, dmoe::kGroupM, tiles,
+                               ws.tile_expert, ws.tile_m0, ws.tile_count};
+    dmoe::launch_permute(pa, stream);
+
+    auto projection = [&](const dmoe::Fp8Proj& w) {
+        dmoe::PackedGroupedArgs a{};
+        a.p.mode = w.wfmt == dmoe::kWfInt4 ? 4 : 5;
+        a.p.w = w.w;
+        a.p.w_se = w.w_se;
+        a.p.w_sn = w.w_sn;
+        a.p.s = reinterpret_cast<const uint8_t*>(w.s);
+        a.p.s_se = w.s_se * 2;
+        a.p.s_sn = w.s_sn * 2;
+        a.p.N = w.N;
+        a.p.K = w.K;
+        a.p.x_row_stride = w.K;
+        a.p.row_div = x.row_div;
+        a.p.order = ws.order;
+        a.p.offsets = ws.offsets;
+        a.p.status = status;
+        a.tile_expert = ws.tile_expert;
+        a.tile_m0 = ws.tile_m0;
+        a.tile_count = ws.tile_count;
+        a.max_tiles = std::min(pairs, tiles);
+        a.gu_dtype = x.x_dtype;
+        return a;
+    };
+    dmoe::PackedGroupedArgs up = projection(g.w13);
+    up.p.gateup = 1;
+    up.p.x = ws.xq;
+    up.p.sa = ws.xs;
+    up.h32 = ws.partial;
+    dmoe::launch_packed_grouped(up, stream);
+    const dmoe::QuantArgs ha{ws.partial, DMOE_F32, g.I, pairs, g.I, 128, 0, ws.hq, ws.hs, status, 1,
+                             ws.offsets + g.experts};
+    dmoe::launch_fp8_quantize(ha, stream);
+
+    dmoe::PackedGroupedArgs dn = projection(g.w2);
+    dn.p.x = ws.hq;
+    dn.hs = ws.hs;
+    dn.p.weighted = 1;
+    dn.p.weights = weights;
+    dn.p.w_dtype = weights_dtype;
+    dn.p.out = out_pairs ? out_pairs : ws.partial;
+    dn.p.out_row_stride = g.H;
+    dmoe::launch_packed_grouped(dn, stream);
+    if (out_pairs) {
+        const dmoe::CombineArgs za{out_pairs, g.H, ids, ids_dtype, g.experts, pairs, 1, g.H, nullptr, DMOE_F32, 0};
+        dmoe::launch_zero_invalid_rows(za, stream);
+    } else {
+        const dmoe::CombineArgs ca{ws.partial, g.H, ids, ids_dtype, g.experts, pairs / top_k, top_k, g.H,
+                                   out, out_dtype, out_row_stride};
+        dmoe::launch_combine(ca, stream);
+    }
+}
+
+// Whether a group-128 call takes the tiled GEMMs: more pairs than one decode
+// call holds (the weights would be read again by every one) and K in whole
+// 256-column steps, within the kernel's 32-bit row offsets.
+bool g128_grouped_fits(const BankGeom& g, int pairs) {
+    auto fits = [](const dmoe::Fp8Proj& w) {
+        return dmoe::packed_grouped_fits(w.wfmt == dmoe::kWfInt4 ? 4 : 5, w.N, w.K, w.w_sn, w.s_sn * 2);
+    };
+    return pairs > dmoe::kMaxDecodePairs && fits(g.w13) && fits(g.w2);
+}
+
+// A group-128 call of any size from route ids (with `ra`: routed first): the
+// tiled GEMMs where they fit and the workspace holds them, else consecutive
+// decode calls of at most kMaxDecodePairs pairs, in order on the stream (pairs
+// of a chunk read rows of their own; layer outputs are cut at whole tokens).
 void g128_forward(const BankGeom& g, const void* x, int x_dtype, int64_t x_row_stride, int rows, int row_div,
                   const void* ids, int ids_dtype, const void* weights, int weights_dtype, int pairs, int top_k,
                   void* out, int out_dtype, int64_t out_row_stride, float* out_pairs, void* workspace,
-                  size_t workspace_bytes, int* status, hipStream_t stream) {
+                  size_t workspace_bytes, int* status, hipStream_t stream, const dmoe::RouteArgs* ra = nullptr) {
     const Activations full{x, x_dtype, x_row_stride, nullptr, nullptr, 0, 0, rows, row_div, g.H};
     check_activations(g, full, pairs);
     // A chunk starts at a row boundary and, for a layer combine, holds whole
@@ -658,6 +755,14 @@ void g128_forward(const BankGeom& g, const void* x, int x_dtype, int64_t x_row_s
         require(top_k <= dmoe::kMaxDecodePairs && row_div % top_k == 0,
                 "group-128 layer call: pairs per row must be a multiple of top_k (at most 256)");
     }
+    if (g128_grouped_fits(g, pairs) &&
+        workspace_bytes >= prefill_workspace_layout(pairs, g.experts, g.H, g.I, nullptr, nullptr, true) &&
+        workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 256 == 0) {
+        g128_grouped_call(g, full, ra, ids, ids_dtype, weights, weights_dtype, pairs, top_k, out, out_dtype,
+                          out_row_stride, out_pairs, workspace, status, stream);
+        return;
+    }
+    if (ra) dmoe::launch_route_topk(*ra, stream);
     const int cap = combine ? (dmoe::kMaxDecodePairs / top_k) * top_k : dmoe::kMaxDecodePairs;
     const int gu_dtype = x_dtype;
     for (int p0 = 0; p0 < pairs;) {
@@ -1210,8 +1315,11 @@ size_t dmoe_quant_workspace_bytes(const DmoeQuantBank* bank, int rows, int pairs
         bank->experts > dmoe::kMaxExperts)
         return 0;
     const int H = std::max(bank->w13.k, bank->w2.n), I = std::max(bank->w2.k, bank->w13.n / 2);
-    if (is_g128_mode(bank->mode))  // consecutive decode calls of at most 256 pairs
-        return fp8_workspace_layout(std::min(pairs, dmoe::kMaxDecodePairs), H, I, nullptr, nullptr);
+    if (is_g128_mode(bank->mode)) {  // decode calls of at most 256 pairs, or the tiled GEMMs
+        const size_t decode = fp8_workspace_layout(std::min(pairs, dmoe::kMaxDecodePairs), H, I, nullptr, nullptr);
+        return pairs <= dmoe::kMaxDecodePairs
+                   ? decode : std::max(decode, prefill_workspace_layout(pairs, bank->experts, H, I, nullptr, nullptr, true));
+    }
     return quant_workspace_layout(rows, pairs, bank->experts, H, I, nullptr, nullptr);
 }
 
@@ -1250,7 +1358,7 @@ int dmoe_quant_projection(const DmoeQuantProj* proj, int experts, int mode, cons
         q.out = out;
         q.out_row_stride = out_row_stride;
         q.status = status;
-        launch_projection(q, std::min(pairs, experts), pairs, st);
+        launch_projection(q, ws, experts, pairs, st);
     });
 }
 
@@ -1308,7 +1416,6 @@ static void quant_forward_impl(const DmoeQuantBank* bank, const void* x, int x_d
             dmoe::launch_route_topk(ra, st);
         }
         if (!small_up || !small_dn) quant_group(ids, ids_dtype, pairs, E, ws, status, st);
-        const int max_active = std::min(pairs, E);
 
         if (small_up) {
             dmoe::QuantGateUpArgs ga{up, x, x_dtype, x_row_stride, rows, row_div, ids, ids_dtype, E, pairs,
@@ -1331,7 +1438,7 @@ static void quant_forward_impl(const DmoeQuantBank* bank, const void* x, int x_d
             up.gateup = 1;
             up.act = ws.act;
             up.status = status;
-            launch_projection(up, max_active, pairs, st);
+            launch_projection(up, ws, E, pairs, st);
         }
 
         if (small_dn) {
@@ -1352,7 +1459,7 @@ static void quant_forward_impl(const DmoeQuantBank* bank, const void* x, int x_d
         dn.out = out_pairs ? out_pairs : ws.partial;
         dn.out_row_stride = H;
         dn.status = status;
-        launch_projection(dn, max_active, pairs, st);
+        launch_projection(dn, ws, E, pairs, st);
 
         if (out_pairs) {
             const dmoe::CombineArgs za{out_pairs, H, ids, ids_dtype, E, pairs, 1, H, nullptr, DMOE_F32, 0};
@@ -1417,16 +1524,15 @@ int dmoe_quant_moe_layer(const DmoeQuantBank* bank, const void* x, int x_dtype, 
                 return;
             }
             // larger calls: the router kernel into the caller's routing outputs,
-            // then the experts over those routes as consecutive decode calls
+            // then the experts over those routes
             const size_t need = fp8_workspace_layout(dmoe::kMaxDecodePairs, g.H, g.I, nullptr, nullptr);
             require(workspace != nullptr && workspace_bytes >= need, "workspace too small");
             require(reinterpret_cast<uintptr_t>(workspace) % 256 == 0, "workspace must be 256-byte aligned");
             const dmoe::RouteArgs ra{logits, logits_row_stride, tokens, g.experts, top_k, renormalize != 0,
                                      ids_out, weights_out, weights_dtype};
-            dmoe::launch_route_topk(ra, st);
             g128_forward(g, x, x_dtype, x_row_stride, tokens, top_k, ids_out, DMOE_I64, weights_out, weights_dtype,
                          pairs, top_k, out, out_dtype, out_row_stride, nullptr, workspace, workspace_bytes, status,
-                         st);
+                         st, &ra);
             return;
         }
         // the experts from routes the call computes first (inside the

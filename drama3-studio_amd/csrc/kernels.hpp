@@ -99,6 +99,8 @@ struct QuantArgs {
     uint8_t* q;             // [rows, cols]
     float* scales;          // [rows, cols / group]
     int* status;
+    int int_order;          // store each 8 bytes in the integer formats' operand order (wfmt.hpp, a_bytes8)
+    const int32_t* valid_rows;  // optional (128-groups): rows past this count are left alone
 };
 
 struct RouteArgs {
@@ -367,6 +369,24 @@ void launch_block_post(const BlockPostArgs& a, int cus, hipStream_t stream);
 // I % 64 == 0, or plain N % 128 == 0.
 bool w4a16_grouped_fits(const QuantProjArgs& a);
 void launch_w4a16_grouped(const QuantProjArgs& a, int max_active, hipStream_t stream, int pairs);
+
+// Tiled grouped projection of modes 1-5 (packed_grouped.hip) over 64-row tiles
+// (kGroupM).  p.order / p.offsets are the permutation, p.active is unused;
+// modes 4, 5: p.s holds fp16 scales (byte strides) and p.sa one scale per FP8
+// activation row of gate/up.
+struct PackedGroupedArgs {
+    QuantProjArgs p;
+    const int32_t* tile_expert;
+    const int32_t* tile_m0;
+    const int32_t* tile_count;
+    int max_tiles;
+    // modes 4, 5
+    int gu_dtype;           // type gate and up are rounded through
+    float* h32;             // gate/up out: silu(gate) * up [sorted position, N / 2]
+    const float* hs;        // down in: the scales [sorted position, K / 128] of the FP8 hidden rows p.x
+};
+bool packed_grouped_fits(int mode, int N, int K, int64_t w_sn, int64_t s_sn);  // byte strides of a row
+void launch_packed_grouped(const PackedGroupedArgs& a, hipStream_t stream);
 
 // Small packed calls (at most 64 route pairs): two launches that group the
 // pairs themselves from the route ids (no permutation launch).

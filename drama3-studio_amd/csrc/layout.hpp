@@ -134,7 +134,9 @@ struct PrefillWorkspace {
     float* partial;
 };
 
-inline PrefillWorkspace prefill_layout(Carver& c, int pairs, int experts, int H, int I) {
+// `partial` also holds the fp32 hidden rows of a group-128 call (h32 true)
+// before the down projection writes it.
+inline PrefillWorkspace prefill_layout(Carver& c, int pairs, int experts, int H, int I, bool h32 = false) {
     PrefillWorkspace w{};
     const int tiles = max_block_tiles(pairs, experts, kGroupM);
     w.head = carve_head(c);
@@ -149,7 +151,7 @@ inline PrefillWorkspace prefill_layout(Carver& c, int pairs, int experts, int H,
     w.xs = c.take<float>("activation scales", (size_t)pairs * (H / 128) * 4);
     w.hq = c.take<uint8_t>("hidden FP8", (size_t)pairs * I);
     w.hs = c.take<float>("hidden scales", (size_t)pairs * (I / 128) * 4);
-    w.partial = c.take<float>("partials fp32", (size_t)pairs * H * 4);
+    w.partial = c.take<float>("partials fp32", (size_t)pairs * (h32 && I > H ? I : H) * 4);
     return w;
 }
 
@@ -177,7 +179,8 @@ inline AlignWorkspace align_layout(Carver& c, int pairs, int experts, int block_
     return w;
 }
 
-// Packed-bank calls: the permutation with its active-expert list, the INT8
+// Packed-bank calls: the permutation with its active-expert list and moe_align
+// tile map, the INT8
 // activation rows (modes 1-3), the bf16 hidden and its INT8 form, and the
 // fp32 partials.
 struct QuantWorkspace {
@@ -187,6 +190,9 @@ struct QuantWorkspace {
     int32_t* counts;
     int32_t* offsets;
     int32_t* active;
+    int32_t* tile_expert;
+    int32_t* tile_m0;
+    int32_t* tile_count;
     int8_t* xq;
     float* xs;
     uint16_t* act;
@@ -197,12 +203,16 @@ struct QuantWorkspace {
 
 inline QuantWorkspace quant_layout(Carver& c, int rows, int pairs, int experts, int H, int I) {
     QuantWorkspace w{};
+    const int tiles = max_block_tiles(pairs, experts, kGroupM);
     w.head = carve_head(c);
     w.permute_scratch = c.take<int32_t>("permute scratch", permute_scratch_bytes(pairs, experts));
     w.order = c.take<int32_t>("order", (size_t)pairs * 4);
     w.counts = c.take<int32_t>("counts", (size_t)experts * 4);
     w.offsets = c.take<int32_t>("offsets", (size_t)(experts + 1) * 4);
     w.active = c.take<int32_t>("active experts", (size_t)(experts + 1) * 4);
+    w.tile_expert = c.take<int32_t>("tile experts", (size_t)tiles * 4);
+    w.tile_m0 = c.take<int32_t>("tile rows", (size_t)tiles * 4);
+    w.tile_count = c.take<int32_t>("tile count", 4);
     w.xq = c.take<int8_t>("activation INT8", (size_t)rows * H);
     w.xs = c.take<float>("activation scales", (size_t)rows * 4);
     w.act = c.take<uint16_t>("hidden bf16", (size_t)pairs * I * 2);

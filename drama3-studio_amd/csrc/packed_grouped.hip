@@ -1,0 +1,352 @@
+// Packed-integer expert banks for many route pairs: tiled grouped GEMMs on
+// 8-bit MFMA operands over the moe_align tile map.  INT8 ConvRot (mode 1), W6A8
+// (2) and W4A8 codebook (3) multiply on i8 MFMA, W4A8-g128 (4) and W6A8-g128
+// (5) on FP8 MFMA, each under the arithmetic of its decode kernels:
+//   modes 1-3: INT8 rows x INT8 weights (decoded exactly as packed_decode.hpp
+//              does), int32 sums, y = bf16(acc * s_a * s_channel); gate/up:
+//              act = bf16(bf16(silu(gate)) * up); down: * route weight (fp32);
+//   modes 4-5: FP8 rows x integer levels exact in E4M3 (wfmt.hpp), per
+//              128-column block acc = fma(dot * s_x, s_w, acc); gate/up rounded
+//              through the compute dtype, h = silu(gate) * up, FP8 per
+//              128-group; down: * route weight (fp32).  In gate/up s_x is
+//              constant along K and multiplies the sum once.
+// Replaces the reference's Triton _quant_gemm over large batches
+// (src/drama_low_vram/quantized_kernels.py:115-214).
+//
+// Workgroup = (64-row tile of one expert's sorted pairs, 128 weight rows), 4
+// waves; a wave owns two 16-row MFMA column tiles (gate/up: 16 gate rows and
+// the matching 16 up rows, so SiLU * up is a register epilogue).  The weight
+// stream bounds these calls, so weights go straight from global memory into
+// the registers of the one wave that uses them and are decoded once per tile;
+// a block's registers take the same block of the next K step as soon as it is
+// decoded.  Activation rows (shared by the waves) go through a double-buffered
+// LDS tile, loaded the same step ahead, one barrier per step.  Row tiles past
+// the expert's last pair are skipped in 16-row units (1 to 4 of them).
+// Modes 4-5 store the hidden fp32; one pass quantizes it for the down kernel.
+//
+// Measured gate/up + down against the column-group kernel (modes 1-3: 16
+// columns a workgroup, 16 rows a pass) and consecutive decode calls (4-5):
+// INT8 197 tokens 276 + 313 -> 90 + 61 us (4.1 TB/s of weights), W6A8 512
+// tokens 201 + 194 -> 112 + 69 us, W6A8-g128 301 tokens 2383 (layer) -> 120 +
+// 64 us.  Decode VALU and its latency bound the 6-bit formats.
+#include <algorithm>
+#include <type_traits>
+
+#include "common.hpp"
+#include "fp8_util.hpp"
+#include "kernels.hpp"
+#include "packed_decode.hpp"
+
+namespace dmoe {
+
+namespace {
+
+// Four waves (128 weight rows): more, smaller workgroups even out the chip's
+// last ones (8 waves measured 97 instead of 67 us for W6A8-g128 down at 301
+// tokens).
+constexpr int kPgWaves = 4, kPgThreads = kPgWaves * kWave;
+constexpr int kPgMaxHiddenBlocks = kMaxInter / 128;
+
+constexpr int pg_sub(int mode, bool gateup) { return mode > 1 && gateup ? 2 : 1; }
+constexpr int pg_groups(int mode, bool gateup) { return pg_sub(mode, gateup) == 2 ? 3 : 4; }
+
+template <int MODE, bool GATEUP>
+struct Fmt {
+    static constexpr bool kFp8 = MODE >= 4;
+    static constexpr int kWf = MODE == 4 ? kWfInt4 : kWfInt6;
+    // pg_sub, pg_groups: 128-column blocks of a K step, workgroups per CU (3: 168 registers, 4:
+    // 128).  Measured for gate/up of the narrow formats (2, 3) 112 / 120 us vs
+    // (1, 4) 127 / 118 (W6A8 at 512 tokens / W6A8-g128 at 301); down 75 / 65.5
+    // vs 68.7 / 63.8; INT8 90.6 + 64.2 vs 89.8 + 60.6 (197 tokens).
+    static constexpr int kSub = pg_sub(MODE, GATEUP);
+    using Acc = std::conditional_t<kFp8, v4f, v4i>;
+};
+
+template <int MODE, bool GATEUP>
+struct alignas(16) PackedLds {
+    uint8_t a[2][Fmt<MODE, GATEUP>::kSub][kGroupM * 128];  // [buffer][128-column block of the step]: swizzled 16-byte chunks
+    int pair[kGroupM];                     // original pair of each tile row (-1: past the expert)
+    float sa[kGroupM], wt[kGroupM];        // its activation scale and route weight
+    // modes 4-5 down: hidden scale of each block and row
+    float rs[MODE >= 4 && !GATEUP ? kPgMaxHiddenBlocks : 1][kGroupM];
+    int8_t tab[MODE == 3 ? 256 * 16 : 16]; // mode 3: INT8 weight of (scale byte, code)
+};
+
+// One lane's weight bytes of one row and 128-column block.
+template <int MODE, bool FP8 = (MODE >= 4)>
+struct BlockRaw {
+    PackedRaw v;
+};
+template <int MODE>
+struct BlockRaw<MODE, true> {
+    WRaw<MODE == 4 ? kWfInt4 : kWfInt6> v;
+    uint32_t scale;  // fp16 bits
+};
+
+// An expert's weights and scales as a wave-uniform base plus 32-bit offsets.
+struct RowBase {
+    const uint8_t *w, *sc;
+};
+
+// 128-column block kb of the row at byte offsets wo (its 16-byte slice grp
+// included) and so: the bytes fetch_wrow / load_wraw give.
+template <int MODE>
+__device__ __forceinline__ BlockRaw<MODE> fetch_block(const RowBase& rb, uint32_t wo, uint32_t ho, uint32_t so, int kb) {
+    BlockRaw<MODE> r;
+    if constexpr (MODE == 1) {
+        const uint8_t* w = rb.w + (wo + (uint32_t)kb * 128u);
+        r.v.a = *(const v4i*)w;
+        r.v.b = *(const v4i*)(w + 16);
+    } else {
+        const v4i lo = *(const v4i*)(rb.w + (wo + (uint32_t)kb * 64u));
+        v2i hi = {0, 0};
+        if constexpr (MODE == 2 || MODE == 5) hi = *(const v2i*)(rb.w + (ho + (uint32_t)kb * 32u));
+        const uint32_t sc = *(const uint16_t*)(rb.sc + (so + (uint32_t)kb * ((MODE >= 4) ? 2u : 8u)));
+        if constexpr (!(MODE >= 4)) {
+            r.v.a = lo;
+            r.v.b = v4i{hi[0], hi[1], 0, 0};
+            r.v.x = sc;
+        } else {
+            if constexpr (MODE == 4) {
+                r.v.v = lo;
+            } else {
+                r.v.lo = lo;
+                r.v.hi = hi;
+            }
+            r.scale = sc;
+        }
+    }
+    return r;
+}
+
+// The tile (m0, mc rows of expert e) x 256 weight rows, MT 16-row units of it.
+template <int MODE, bool GATEUP, int MT>
+__device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLds<MODE, GATEUP>& s, int e, int m0, int mc) {
+    using F = Fmt<MODE, GATEUP>;
+    constexpr int kSub = F::kSub;
+    const QuantProjArgs& p = a.p;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int col = lane % 16, grp = lane / 16;
+    const int half = p.N / 2, KB = p.K / 128, steps = KB / kSub;
+    // this lane's two weight rows (rows past the matrix repeat its last; not stored)
+    const int n0 = GATEUP ? blockIdx.y * (kPgWaves * 16) + wave * 16 + col : blockIdx.y * (kPgWaves * 32) + wave * 32 + col;
+    int n[2];
+    n[0] = min(n0, (GATEUP ? half : p.N) - 1);
+    n[1] = GATEUP ? half + n[0] : min(n0 + 16, p.N - 1);
+    // activation chunks of this thread: 16 bytes of tile rows ar + q * kRowStep
+    // (rows past the last pair repeat it)
+    constexpr int kRowStep = kPgThreads / 8, kChunks = (16 * MT + kRowStep - 1) / kRowStep;
+    const int ar = threadIdx.x / 8, ac = threadIdx.x % 8;
+    constexpr bool kByPosition = F::kFp8 && !GATEUP;  // the FP8 hidden rows lie in sorted order
+    const uint8_t* asrc[kChunks];
+#pragma unroll
+    for (int q = 0; q < kChunks; ++q) {
+        const int pos = m0 + min(ar + q * kRowStep, mc - 1);
+        asrc[q] = (const uint8_t*)p.x + (int64_t)(kByPosition ? pos : p.order[pos] / p.row_div) * p.x_row_stride + ac * 16;
+    }
+    const int aoff = ar * 128 + ((ac ^ (ar % 8)) * 16);  // kRowStep is a multiple of 8: the same swizzle
+    const RowBase rb{p.w + (int64_t)e * p.w_se, p.s + (int64_t)e * p.s_se};
+    uint32_t wo[2], so[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        wo[c] = (uint32_t)n[c] * (uint32_t)p.w_sn + grp * (MODE == 1 ? 32 : 16);
+        so[c] = (uint32_t)n[c] * (uint32_t)p.s_sn + (F::kFp8 ? 0 : grp * 2);
+    }
+    const uint32_t high = p.K / 2 - grp * 8;  // from a row's low slice to its 2-bit high slice (grp * 16 -> + grp * 8)
+
+    v4i areg[kSub][kChunks];
+    BlockRaw<MODE> raw[kSub][2];  // [block][row]
+    auto load_a = [&](int st) {
+#pragma unroll
+        for (int b = 0; b < kSub; ++b)
+#pragma unroll
+            for (int q = 0; q < kChunks; ++q) areg[b][q] = *(const v4i*)(asrc[q] + (st * kSub + b) * 128);
+    };
+    auto stage_a = [&](int buf) {
+#pragma unroll
+        for (int b = 0; b < kSub; ++b)
+#pragma unroll
+            for (int q = 0; q < kChunks; ++q) *(v4i*)&s.a[buf][b][aoff + q * kRowStep * 128] = areg[b][q];
+    };
+    auto load_b = [&](int st, int b, int c) { raw[b][c] = fetch_block<MODE>(rb, wo[c], wo[c] + high, so[c], st * kSub + b); };
+    typename F::Acc acc[MT][2];
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi) acc[mi][0] = acc[mi][1] = typename F::Acc{0, 0, 0, 0};
+
+    // Multiply step st; a weight block's registers take the same block of step
+    // `next` as soon as it is decoded.
+    auto compute = [&](int st, int next, int buf) {
+        const int o0 = ((2 * grp) ^ (col % 8)) * 16, o1 = ((2 * grp + 1) ^ (col % 8)) * 16;
+#pragma unroll
+        for (int b = 0; b < kSub; ++b) {
+            const uint8_t* at = s.a[buf][b] + col * 128;
+            __builtin_amdgcn_sched_barrier(0);  // one block's operands live at a time
+            if constexpr (!F::kFp8) {
+                PackedRow w[2];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    if constexpr (MODE == 3) decode_w4a8_tab(raw[b][c].v, s.tab, w[c]);
+                    else decode_wrow<MODE, false>(raw[b][c].v, n[c], nullptr, w[c]);
+                    load_b(next, b, c);
+                }
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi) {
+                    const v4i a0 = *(const v4i*)(at + mi * 16 * 128 + o0), a1 = *(const v4i*)(at + mi * 16 * 128 + o1);
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        acc[mi][c] = mfma_i8(a0, w[c].r[0], acc[mi][c]);
+                        acc[mi][c] = mfma_i8(a1, w[c].r[1], acc[mi][c]);
+                    }
+                }
+            } else {
+                const v4f zero = {0, 0, 0, 0};
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const float sw = f16_to_f32((uint16_t)raw[b][c].scale);
+                    v8i lo, hi;
+                    if (c > 0) __builtin_amdgcn_sched_barrier(0);
+                    expand_w<F::kWf>(raw[b][c].v, lo, hi);
+                    load_b(next, b, c);
+#pragma unroll
+                    for (int mi = 0; mi < MT; ++mi) {
+                        const v4i a0 = *(const v4i*)(at + mi * 16 * 128 + o0), a1 = *(const v4i*)(at + mi * 16 * 128 + o1);
+                        const v8i av = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+                        v4f rs = {1.0f, 1.0f, 1.0f, 1.0f};
+                        if constexpr (!GATEUP) rs = *(const v4f*)&s.rs[st * kSub + b][16 * mi + 4 * grp];
+                        v4f d = mfma_fp8(av, lo, zero);
+                        if constexpr (MODE == 5) d = mfma_fp8(av, hi, d);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float t = GATEUP ? d[i] : d[i] * rs[i];
+                            acc[mi][c][i] = fmaf(t, sw, acc[mi][c][i]);
+                        }
+                    }
+                }
+            }
+        }
+    };
+
+    load_a(0);
+#pragma unroll
+    for (int b = 0; b < kSub; ++b)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) load_b(0, b, c);
+    if (threadIdx.x < kGroupM) {
+        const int r = threadIdx.x, pr = p.order[m0 + min(r, mc - 1)];
+        s.pair[r] = r < mc ? pr : -1;
+        if (p.sa) s.sa[r] = p.sa[pr / p.row_div];
+        if (p.weighted) s.wt[r] = load_as_f32(p.weights, pr, p.w_dtype);
+    }
+    if constexpr (MODE == 3) {  // entry 16 * scale byte + code; a thread's entries share the code
+        const float level = *(const float*)(p.s + (int64_t)e * p.s_se + (int64_t)(threadIdx.x % 16) * p.s_sn + p.K / 16 + 4);
+        for (int i = threadIdx.x; i < 256 * 16; i += kPgThreads) s.tab[i] = q8(level, e4m3((uint32_t)i / 16));
+    }
+    if constexpr (F::kFp8 && !GATEUP) {
+        for (int i = threadIdx.x; i < kGroupM * KB; i += kPgThreads) {
+            const int r = i / KB, kb = i % KB;
+            s.rs[kb][r] = a.hs[(int64_t)(m0 + min(r, mc - 1)) * KB + kb];
+        }
+    }
+    stage_a(0);
+    // The barrier makes this step's activation rows visible; the buffer staged
+    // into was read before it.  The last step loads itself again: no branch
+    // around the loads, so the waits stay counted and never drain them.
+    for (int st = 0, buf = 0; st < steps; ++st, buf ^= 1) {
+        const int next = min(st + 1, steps - 1);
+        load_a(next);
+        lds_barrier();
+        compute(st, next, buf);
+        stage_a(buf ^ 1);
+    }
+
+    // epilogue: a lane holds column `col` of each 16 x 16 result, rows 4 grp + i
+    {
+        float sb[2] = {1.0f, 1.0f};
+        if constexpr (!F::kFp8) {
+            sb[0] = channel_scale<MODE>(p, e, n[0]);
+            sb[1] = channel_scale<MODE>(p, e, n[1]);
+        }
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = 16 * mi + 4 * grp + i, pr = s.pair[r];
+                if (pr < 0) continue;
+                float y[2];
+                const float sa = F::kFp8 && !GATEUP ? 1.0f : s.sa[r];
+                if constexpr (F::kFp8) {
+                    y[0] = acc[mi][0][i] * sa;
+                    y[1] = acc[mi][1][i] * sa;
+                } else {
+                    y[0] = bf16_round((float)acc[mi][0][i] * sa * sb[0]);
+                    y[1] = bf16_round((float)acc[mi][1][i] * sa * sb[1]);
+                }
+                if constexpr (GATEUP && F::kFp8) {
+                    const float h = silu_f32(round_through(y[0], a.gu_dtype)) * round_through(y[1], a.gu_dtype);
+                    if (n0 < half) a.h32[(int64_t)(m0 + r) * half + n0] = h;
+                } else if constexpr (GATEUP) {
+                    const float act = bf16_round(bf16_round(y[0] / (1.0f + expf(-y[0]))) * y[1]);
+                    if (n0 < half) p.act[(int64_t)pr * half + n0] = __builtin_bit_cast(uint16_t, (__bf16)act);
+                } else {
+                    const float wt = s.wt[r];
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const int nc = n0 + 16 * c;
+                        if (nc >= p.N) continue;
+                        const int64_t o = (int64_t)pr * p.out_row_stride + nc;
+                        if (p.weighted) ((float*)p.out)[o] = y[c] * wt;
+                        else ((uint16_t*)p.out)[o] = __builtin_bit_cast(uint16_t, (__bf16)y[c]);
+                    }
+                }
+            }
+        }
+    }
+}
+
+template <int MODE, bool GATEUP>
+__global__ __launch_bounds__(kPgThreads, pg_groups(MODE, GATEUP)) void packed_grouped_kernel(PackedGroupedArgs a) {
+    __shared__ PackedLds<MODE, GATEUP> s;
+    const int tile = blockIdx.x;
+    if (tile >= *a.tile_count) return;
+    const int e = __builtin_amdgcn_readfirstlane(a.tile_expert[tile]);
+    const int m0 = __builtin_amdgcn_readfirstlane(a.tile_m0[tile]);
+    const int mc = min(kGroupM, a.p.offsets[e + 1] - m0);
+    if (mc <= 16) packed_tile<MODE, GATEUP, 1>(a, s, e, m0, mc);
+    else if (mc <= 32) packed_tile<MODE, GATEUP, 2>(a, s, e, m0, mc);
+    else if (mc <= 48) packed_tile<MODE, GATEUP, 3>(a, s, e, m0, mc);
+    else packed_tile<MODE, GATEUP, 4>(a, s, e, m0, mc);
+}
+
+}  // namespace
+
+// Whole K steps, and an expert's rows within 32-bit byte offsets.
+bool packed_grouped_fits(int mode, int N, int K, int64_t w_sn, int64_t s_sn) {
+    return mode >= 1 && mode <= 5 && K % (mode == 1 ? 128 : 256) == 0 && N * w_sn < (int64_t(1) << 32) &&
+           N * s_sn < (int64_t(1) << 32);
+}
+
+template <int MODE, bool GATEUP>
+static void launch_mode(const PackedGroupedArgs& a, hipStream_t stream) {
+    constexpr int kCols = kPgWaves * (GATEUP ? 16 : 32);
+    const int cols = ((GATEUP ? a.p.N / 2 : a.p.N) + kCols - 1) / kCols;
+    // a multiple of the 8 XCDs: the column tiles of a row tile share its XCD's L2
+    const dim3 grid((unsigned)((a.max_tiles + 7) / 8 * 8), (unsigned)cols);
+    hipLaunchKernelGGL((packed_grouped_kernel<MODE, GATEUP>), grid, dim3(kPgThreads), 0, stream, a);
+}
+
+void launch_packed_grouped(const PackedGroupedArgs& a, hipStream_t stream) {
+    auto go = [&](auto gateup) {
+        constexpr bool kGateUp = decltype(gateup)::value;
+        switch (a.p.mode) {
+            case 1: launch_mode<1, kGateUp>(a, stream); break;
+            case 2: launch_mode<2, kGateUp>(a, stream); break;
+            case 3: launch_mode<3, kGateUp>(a, stream); break;
+            case 4: launch_mode<4, kGateUp>(a, stream); break;
+            default: launch_mode<5, kGateUp>(a, stream); break;
+        }
+    };
+    if (a.p.gateup) go(std::true_type{});
+    else go(std::false_type{});
+}
+
+}  // namespace dmoe

@@ -30,6 +30,7 @@
 #include "common.hpp"
 #include "handoff.hpp"
 #include "kernels.hpp"
+#include "packed_decode.hpp"
 #include "route.hpp"
 
 namespace dmoe {
@@ -39,28 +40,6 @@ namespace {
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int kQWaves = 8, kQThreads = kQWaves * kWave;
-
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-    const v2bf p = {(__bf16)a, (__bf16)b};
-    return __builtin_bit_cast(uint32_t, p);
-}
-
-__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
-    return (uint32_t)f32_to_f16(a) | ((uint32_t)f32_to_f16(b) << 16);
-}
-
-__device__ __forceinline__ float bf16_round(float v) { return (float)(__bf16)v; }
-
-// E4M3 byte -> fp32 (hardware decode of one byte).
-__device__ __forceinline__ float e4m3(uint32_t byte) { return fp8x2_to_f32(byte & 0xFFu, false)[0]; }
-
-using h2v = _Float16 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ int8_t q8(float level, float rel) {
-    const float v = fminf(fmaxf(__builtin_rintf(level * rel), -127.0f), 127.0f);
-    return (int8_t)(int)v;
-}
 
 struct QuantLds {
     float red[kQWaves][kWave][8];  // cross-wave reduction (fp32 or int32 bits)
@@ -196,154 +175,6 @@ void launch_rotate_quant(const RotateArgs& a, hipStream_t stream) {
 
 // ------------------------------------------------------------- projection
 
-// Dequantized operand registers of one weight row for one 128-K block.
-struct WRow {
-    v4i r[4];  // mode 0: 4 x (8 bf16 / fp16); modes 1-3: r[0], r[1] = 2 x 16 int8
-};
-
-// Zero-point word of banks without qzeros (zero point 8 in every nibble), so
-// the mode-0 fetch loads a word either way.
-__device__ int32_t g_zero_point8 = (int32_t)0x88888888u;
-
-// The bytes a lane loads for one weight row's 128-K block (its 32 K values),
-// kept apart from the dequantization so loads can be issued early.
-struct WRaw {
-    v4i a;       // mode 0: 4 code words; mode 1: int8 bytes 0..15; modes 2, 3: low-nibble words
-    v4i b;       // mode 1: int8 bytes 16..31; mode 2: b[0], b[1] = 2-bit high planes
-    uint32_t x;  // mode 0: fp16 scale bits; modes 2, 3: the two e4m3 rel bytes
-    uint32_t z;  // mode 0: qzeros word (0x88888888: zero point 8)
-};
-
-template <int MODE>
-__device__ __forceinline__ WRaw fetch_wrow(const QuantProjArgs& a, int e, int n, int kb, int grp) {
-    const uint8_t* w = a.w + (int64_t)e * a.w_se + (int64_t)n * a.w_sn;
-    const uint8_t* sc = a.s + (int64_t)e * a.s_se + (int64_t)n * a.s_sn;
-    WRaw r{};
-    if constexpr (MODE == 0) {
-        r.a = *(const v4i*)(w + kb * 64 + grp * 16);
-        r.x = *(const uint16_t*)(sc + kb * 2);
-        const int32_t* zw = a.z ? a.z + (int64_t)e * a.z_se + (int64_t)kb * (a.N / 8) + n / 8 : &g_zero_point8;
-        r.z = (uint32_t)*zw;
-    } else if constexpr (MODE == 1) {
-        r.a = *(const v4i*)(w + kb * 128 + grp * 32);
-        r.b = *(const v4i*)(w + kb * 128 + grp * 32 + 16);
-    } else {
-        // 32 codes: low nibbles (16 bytes), mode 2 also 2-bit high parts (8 bytes)
-        r.a = *(const v4i*)(w + kb * 64 + grp * 16);
-        if constexpr (MODE == 2) {
-            const uint2 high = *(const uint2*)(w + a.K / 2 + kb * 32 + grp * 8);
-            r.b[0] = (int)high.x;
-            r.b[1] = (int)high.y;
-        }
-        r.x = *(const uint16_t*)(sc + kb * 8 + grp * 2);
-    }
-    return r;
-}
-
-template <int MODE, bool F16>
-__device__ __forceinline__ void decode_wrow(const WRaw& raw, int n, const float* book, WRow& out) {
-    if constexpr (MODE == 0) {
-        const float scale = f16_to_f32((uint16_t)raw.x);
-        const int zp = (int)((raw.z >> (4 * (n % 8))) & 15u);
-        const float bias = -(float)zp * scale;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const uint32_t u = (uint32_t)raw.a[t];
-            float v[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = fmaf((float)((u >> (4 * i)) & 15u), scale, bias);  // exact
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                out.r[t][i] = (int)(F16 ? pack_f16(v[2 * i], v[2 * i + 1]) : pack_bf16(v[2 * i], v[2 * i + 1]));
-        }
-    } else if constexpr (MODE == 1) {
-        out.r[0] = raw.a;
-        out.r[1] = raw.b;
-    } else if constexpr (MODE == 2) {
-        // Two codes per packed fp16 pair: code c as the fp16 1024 + c (exponent
-        // 2^10, ulp 1); level = that - 1056; level * rel is exact (6 + 4
-        // significant bits, |.| <= 32 * 448); clamping to [-127, 127] before
-        // the rounding equals clamping after it (integer bounds); + 1536 then
-        // rounds to the nearest even integer r and leaves r's two's-complement
-        // byte as the low byte of the half -- q8(level, rel) for every code and
-        // E4M3 byte.  Pair k of a group holds codes k (low half) and k + 8.
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {  // 16 codes = K [32 g + 16 j, +16): one rel group
-            const _Float16 rh = (_Float16)e4m3(raw.x >> (8 * j));  // exact
-            const h2v rel2 = {rh, rh};
-            const uint32_t a0 = (uint32_t)raw.a[2 * j], a1 = (uint32_t)raw.a[2 * j + 1], hw = (uint32_t)raw.b[j];
-            uint32_t pr[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t lo = ((a0 >> (4 * k)) & 15u) | (((a1 >> (4 * k)) & 15u) << 16);
-                const uint32_t hi = (hw >> (2 * k)) & 0x00030003u;
-                h2v v = (__builtin_bit_cast(h2v, lo | (hi << 4) | 0x64006400u) - h2v{1056, 1056}) * rel2;
-                v = __builtin_elementwise_min(__builtin_elementwise_max(v, h2v{-127, -127}), h2v{127, 127});
-                pr[k] = __builtin_bit_cast(uint32_t, v + h2v{1536, 1536});
-            }
-            // int q of the group: codes 4q .. 4q + 3 (low bytes of the halves)
-            const uint32_t t01 = __builtin_amdgcn_perm(pr[1], pr[0], 0x06020400u);
-            const uint32_t t23 = __builtin_amdgcn_perm(pr[3], pr[2], 0x06020400u);
-            const uint32_t t45 = __builtin_amdgcn_perm(pr[5], pr[4], 0x06020400u);
-            const uint32_t t67 = __builtin_amdgcn_perm(pr[7], pr[6], 0x06020400u);
-            out.r[j][0] = (int)__builtin_amdgcn_perm(t23, t01, 0x05040100u);
-            out.r[j][1] = (int)__builtin_amdgcn_perm(t67, t45, 0x05040100u);
-            out.r[j][2] = (int)__builtin_amdgcn_perm(t23, t01, 0x07060302u);
-            out.r[j][3] = (int)__builtin_amdgcn_perm(t67, t45, 0x07060302u);
-        }
-    } else {
-        const float rel[2] = {e4m3(raw.x), e4m3(raw.x >> 8)};
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {  // 16 codes = K [32 g + 16 j, +16): one rel group
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {  // 4 codes per output int
-                uint32_t packed = 0;
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const int c = j * 16 + q * 4 + b;  // code index within the lane's 32
-                    const uint32_t lo = ((uint32_t)raw.a[c / 8] >> (4 * (c % 8))) & 15u;
-                    packed |= ((uint32_t)(uint8_t)q8(book[lo], rel[j])) << (8 * b);
-                }
-                out.r[j][q] = (int)packed;
-            }
-        }
-    }
-}
-
-template <int MODE, bool F16>
-__device__ __forceinline__ void load_wrow(const QuantProjArgs& a, int e, int n, int kb, int grp, const float* book,
-                                          WRow& out) {
-    decode_wrow<MODE, F16>(fetch_wrow<MODE>(a, e, n, kb, grp), n, book, out);
-}
-
-// W4A8 INT8 weights by table: tab[rel byte * 16 + code] = q8(book[code],
-// e4m3(rel byte)), so the result equals decode_wrow<3>'s.  A lane's four codes
-// of an output int index the 16-byte row of its group's scale byte through
-// two byte permutes (codes 0-7 and 8-15) and a byte select.
-__device__ __forceinline__ void decode_w4a8_tab(const WRaw& raw, const int8_t* tab, WRow& out) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {  // 16 codes = K [32 g + 16 j, +16): one rel group
-        const v4i row = *(const v4i*)(tab + (((uint32_t)raw.x >> (8 * j)) & 0xFFu) * 16);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {  // codes 16 j + 4 q .. +3: nibbles 4 (q % 2) .. +3 of word 2 j + q / 2
-            uint32_t t = ((uint32_t)raw.a[2 * j + q / 2] >> (16 * (q % 2))) & 0xFFFFu;
-            t = (t | (t << 8)) & 0x00FF00FFu;
-            t = (t | (t << 4)) & 0x0F0F0F0Fu;  // byte b: code 4 q + b
-            const uint32_t sel = t & 0x07070707u, high = ((t >> 3) & 0x01010101u) * 0xFFu;
-            const uint32_t lo8 = __builtin_amdgcn_perm((uint32_t)row[1], (uint32_t)row[0], sel);
-            const uint32_t hi8 = __builtin_amdgcn_perm((uint32_t)row[3], (uint32_t)row[2], sel);
-            out.r[j][q] = (int)((hi8 & high) | (lo8 & ~high));
-        }
-    }
-}
-
-template <int MODE>
-__device__ __forceinline__ float channel_scale(const QuantProjArgs& a, int e, int n) {
-    const uint8_t* sc = a.s + (int64_t)e * a.s_se + (int64_t)n * a.s_sn;
-    if constexpr (MODE == 1) return *(const float*)sc;
-    else return *(const float*)(sc + a.K / 16);
-}
-
 // KBW = 128-column K blocks per wave (K <= 8 * 128 * KBW, K <= kMaxQuantK).
 template <int MODE, bool GATEUP, bool F16, int KBW>
 __global__ __launch_bounds__(kQThreads) void quant_proj_kernel(QuantProjArgs a) {
@@ -365,7 +196,7 @@ __global__ __launch_bounds__(kQThreads) void quant_proj_kernel(QuantProjArgs a) 
     }
 
     // this wave's weight rows, dequantized once
-    WRow bg[KBW], bu[KBW];
+    PackedRow bg[KBW], bu[KBW];
 #pragma unroll
     for (int i = 0; i < KBW; ++i) {
         const int kb = wave + i * kQWaves;
@@ -769,7 +600,7 @@ __device__ __forceinline__ void quant_gateup_body(const QuantGateUpArgs& a, QGat
     const int nxg = n0 + 16 + (col & 7), nxu = I + nxg, nx = col < 8 ? nxg : nxu;  // third tile (NT 3)
 
     // weight rows of this wave, loaded now, dequantized after the rotation
-    WRaw rg[KBW], ru[KBW], rx[NX];
+    PackedRaw rg[KBW], ru[KBW], rx[NX];
 #pragma unroll
     for (int i = 0; i < KBW; ++i) {
         const int kb = min(wave + i * kQWaves, KB - 1);  // blocks past K: loaded, never used
@@ -827,7 +658,7 @@ __device__ __forceinline__ void quant_gateup_body(const QuantGateUpArgs& a, QGat
     }
     lds_barrier();
 
-    WRow bg[KBW], bu[KBW], bx[NX];
+    PackedRow bg[KBW], bu[KBW], bx[NX];
 #pragma unroll
     for (int i = 0; i < KBW; ++i) {
         const int kb = wave + i * kQWaves;
@@ -1071,7 +902,7 @@ struct PackedHidden {
 template <int KB2>
 struct DownBatch {
     int e0, e1, e, ec;
-    WRaw raw[KB2];
+    PackedRaw raw[KB2];
     float sch, bk;
 };
 template <int MODE, int KB2>
@@ -1158,7 +989,7 @@ __device__ __forceinline__ void quant_down_body(const QuantDownArgs& a, QDownLds
     const int n = n0 + (col & 7);
     DownBatch<KB2> cur;
     auto fetch_batch = [&](int bi) { fetch_down_batch<MODE, KB2>(w, g, bi, n, cur); };
-    WRow b[KB2];
+    PackedRow b[KB2];
     auto decode_batch = [&]() {
         if constexpr (MODE == 3) {
             if (lane < 32) s.book[wave][lane / 16][lane % 16] = cur.bk;  // read back by this wave only

@@ -20,10 +20,14 @@ namespace dmoe {
 // One 16-lane row per 128-group (8 values per lane, DPP max); for one scale
 // per row the 256-thread block reduces the row.  With `silu_mul` the row holds
 // gate|up and silu(gate) * up is quantized.
+__device__ __forceinline__ uint64_t stored_order(const QuantArgs& a, uint64_t v) {
+    return a.int_order ? a_bytes8<kWfInt4>(v) : v;
+}
+
 __device__ void quantize_unit128(const QuantArgs& a, int64_t unit) {
     const int col = threadIdx.x % 16;
     const int groups = a.cols / 128;
-    const bool live = unit < (int64_t)a.rows * groups;
+    const bool live = unit < (int64_t)(a.valid_rows ? min(*a.valid_rows, a.rows) : a.rows) * groups;
     const int64_t row = live ? unit / groups : 0, c0 = live ? (unit % groups) * 128 : 0;
     const int64_t base = row * a.x_row_stride;
     F8 v;
@@ -36,7 +40,7 @@ __device__ void quantize_unit128(const QuantArgs& a, int64_t unit) {
     }
     const float scale = fmaxf(row_max(absmax8(v, live ? a.status : nullptr)), 1e-10f) * (1.0f / 448.0f);
     if (live) {
-        *(uint64_t*)(a.q + row * a.cols + c0 + col * 8) = encode8(v, scale);
+        *(uint64_t*)(a.q + row * a.cols + c0 + col * 8) = stored_order(a, encode8(v, scale));
         if (col == 0) a.scales[row * groups + c0 / 128] = scale;
     }
 }
@@ -53,7 +57,7 @@ __device__ void quantize_row(const QuantArgs& a, int64_t row) {
     amax = fmaxf(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])), 1e-10f);
     const float scale = amax * (1.0f / 448.0f);
     for (int c = threadIdx.x * 8; c < a.cols; c += 256 * 8)
-        *(uint64_t*)(a.q + row * a.cols + c) = encode8(load8(a.x, base + c, a.x_dtype), scale);
+        *(uint64_t*)(a.q + row * a.cols + c) = stored_order(a, encode8(load8(a.x, base + c, a.x_dtype), scale));
     if (threadIdx.x == 0) a.scales[row] = scale;
 }
 

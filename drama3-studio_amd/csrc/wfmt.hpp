@@ -173,24 +173,18 @@ __device__ __forceinline__ uint64_t a_bytes8(uint64_t v) {
     }
 }
 
-// c + A * W over one 128-column block: A from a_operand<WF>, W the raw slice.
+// A raw integer slice as FP8 MFMA B operands: 4 bits one (lo), 6 bits two whose
+// products add (lo + hi).
 template <int WF>
-__device__ __forceinline__ v4f mfma_w(const v8i& a, const WRaw<WF>& w, const v4f& c) {
-    if constexpr (WF == kWfFp8) {
-        return mfma_fp8(a, w.v, c);
-    } else if constexpr (WF == kWfInt4) {
-        v8i b;
+__device__ __forceinline__ void expand_w(const WRaw<WF>& w, v8i& lo, v8i& hi) {
+    static_assert(WF != kWfFp8, "integer formats");
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (WF == kWfInt4) {
             const v2i p = expand_nibbles<kInt4T0, kInt4T1, kInt4T2, kInt4T3>((uint32_t)w.v[i]);
-            b[2 * i] = p[0];
-            b[2 * i + 1] = p[1];
-        }
-        return mfma_fp8(a, b, c);
-    } else {
-        v8i lo, hi;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
+            lo[2 * i] = p[0];
+            lo[2 * i + 1] = p[1];
+        } else {
             const v2i l = expand_nibbles<kLowT0, kLowT1, kLowT2, kLowT3>((uint32_t)w.lo[i]);
             const v2i h = expand_high(((uint32_t)w.hi[i / 2] >> (16 * (i % 2))) & 0xFFFFu);
             lo[2 * i] = l[0];
@@ -198,7 +192,19 @@ __device__ __forceinline__ v4f mfma_w(const v8i& a, const WRaw<WF>& w, const v4f
             hi[2 * i] = h[0];
             hi[2 * i + 1] = h[1];
         }
-        return mfma_fp8(a, hi, mfma_fp8(a, lo, c));
+    }
+}
+
+// c + A * W over one 128-column block: A from a_operand<WF>, W the raw slice.
+template <int WF>
+__device__ __forceinline__ v4f mfma_w(const v8i& a, const WRaw<WF>& w, const v4f& c) {
+    if constexpr (WF == kWfFp8) {
+        return mfma_fp8(a, w.v, c);
+    } else {
+        v8i lo, hi;
+        expand_w<WF>(w, lo, hi);
+        if constexpr (WF == kWfInt4) return mfma_fp8(a, lo, c);
+        else return mfma_fp8(a, hi, mfma_fp8(a, lo, c));
     }
 }
 

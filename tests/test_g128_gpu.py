@@ -267,3 +267,31 @@ def test_g128_layer_combine_with_pairs_per_row_not_top_k(cuda, mode):
                                                  w[p:p + 1].numpy(), x_group=512) for p in range(pairs)])
     expected = parts.reshape(tokens, top_k, 512).sum(1)
     assert rel_inf(out.cpu().numpy(), expected) < TOL
+
+
+@pytest.mark.parametrize("mode", [4, 5])
+@pytest.mark.parametrize("hidden,inter", [(256, 512), (512, 256), (256, 384)])
+def test_g128_tiled_row_edges(cuda, mode, hidden, inter):
+    """More pairs than one decode call: the tiled GEMMs with experts of 1, 16,
+    17, 32, 33, 48, 49, 64, 65 and 0 rows, invalid ids and an intermediate size
+    above and below the hidden one; inter 384 is no whole K step and runs as
+    consecutive decode calls."""
+    print_case("g128 tiled edges", mode, hidden, inter)
+    counts = [1, 16, 17, 32, 33, 0, 48, 49, 64, 65]
+    store = bank_on(cuda, mode, len(counts), hidden, inter, 11 + mode)
+    g = torch.Generator().manual_seed(mode * inter)
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    ids = flat[torch.randperm(len(flat), generator=g)][:, None]
+    ids[5, 0], ids[280, 0] = -2, len(counts)
+    x = torch.randn(len(ids), hidden, generator=g).bfloat16()
+    w = torch.rand(len(ids), 1, generator=g) + 0.1
+    backend = QuantizedExpertBackend(mode)
+    backend.status(cuda)
+    out = backend.forward_pairs(x.to(cuda), ids.to(cuda), w.to(cuda), store)
+    assert backend.status(cuda) == _lib.STATUS_BAD_EXPERT_ID
+    assert torch.count_nonzero(out[5]) == 0 and torch.count_nonzero(out[280]) == 0
+    keep = [r for r in range(len(ids)) if r not in (5, 280)]
+    b13, b2 = oracle_banks(store)
+    expected = np.concatenate([orc.fp8_expert_pairs(b13, b2, x[r].float().numpy(), ids[r].numpy(), w[r].numpy(),
+                                                    x_group=hidden) for r in keep])
+    assert rel_inf(out.cpu().numpy()[keep], expected) < TOL

@@ -370,3 +370,28 @@ def test_gptq_linear_matches_dequantize_then_matmul(cuda, rows, n, k, x_dtype):
     matrix = torch_cpu.dequantize(0, words.T.contiguous(), scales.T.contiguous(), k, x_dtype)
     expected = (x.float() @ matrix.T).bfloat16().float()
     assert rel_inf(out.reshape(rows, n).float().cpu().numpy(), expected.numpy()) < 5e-3
+
+
+@pytest.mark.parametrize("mode", [1, 2, 3])
+@pytest.mark.parametrize("n,k,weighted", [(144, 256, True), (16, 1024, False)])
+def test_tiled_projection_row_and_column_edges(cuda, mode, n, k, weighted):
+    """The tiled 8-bit GEMM where its tiles end: experts of 1, 16, 17, 32, 33,
+    48, 49, 64, 65 and 0 rows, invalid ids, N past the last whole column tile
+    and below one.  INT32 sums and the two scale products are exact restatements
+    of the oracle's, so bf16 results differ by rounding ties only."""
+    print_case("tiled projection edges", mode, n, k, weighted)
+    g = torch.Generator().manual_seed(10 * mode + n)
+    counts = [1, 16, 17, 32, 33, 0, 48, 49, 64, 65]
+    store = random_quantized_bank(mode, len(counts), k, max(256, n), generator=g)
+    bank, scales = store.w13_weight[:, :n], store.w13_scale_inv[:, :n]
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    ids = flat[torch.randperm(len(flat), generator=g)]
+    ids[3], ids[200] = -1, len(counts)
+    x = torch.randn(len(ids), k, generator=g).bfloat16()
+    w = torch.rand(len(ids), generator=g) + 0.1
+    out = quantized.projection(x.to(cuda), ids.to(cuda), w.to(cuda), bank.to(cuda), scales.to(cuda), mode=mode,
+                               weighted=weighted)
+    keep = [r for r in range(len(ids)) if 0 <= int(ids[r]) < len(counts)]
+    b = orc.QuantBank(mode, bank.contiguous().numpy(), scales.contiguous().numpy(), n, k)
+    expected = orc.quant_projection(b, x.float().numpy()[keep], ids.numpy()[keep], w.numpy()[keep], weighted=weighted)
+    assert rel_inf(out.float().cpu().numpy()[keep], expected) < 2.0 ** -8
