@@ -24,7 +24,7 @@
 // the expert's last pair are skipped in 16-row units (1 to 4 of them).
 // Modes 4-5 store the hidden fp32; one pass quantizes it for the down kernel.
 //
-// Measured gate/up + down against the column-group kernel (modes 1-3: 16
+// Measured (first form) gate/up + down against the column-group kernel (modes 1-3: 16
 // columns a workgroup, 16 rows a pass) and consecutive decode calls (4-5):
 // INT8 197 tokens 276 + 313 -> 90 + 61 us (4.1 TB/s of weights), W6A8 512
 // tokens 201 + 194 -> 112 + 69 us, W6A8-g128 301 tokens 2383 (layer) -> 120 +
@@ -47,17 +47,17 @@ namespace {
 constexpr int kPgWaves = 4, kPgThreads = kPgWaves * kWave;
 constexpr int kPgMaxHiddenBlocks = kMaxInter / 128;
 
-constexpr int pg_sub(int mode, bool gateup) { return mode > 1 && gateup ? 2 : 1; }
+constexpr int pg_sub(int mode, bool gateup) { return (mode == 2 || mode == 3) && gateup ? 2 : 1; }
 constexpr int pg_groups(int mode, bool gateup) { return pg_sub(mode, gateup) == 2 ? 3 : 4; }
 
 template <int MODE, bool GATEUP>
 struct Fmt {
     static constexpr bool kFp8 = MODE >= 4;
     static constexpr int kWf = MODE == 4 ? kWfInt4 : kWfInt6;
-    // pg_sub, pg_groups: 128-column blocks of a K step, workgroups per CU (3: 168 registers, 4:
-    // 128).  Measured for gate/up of the narrow formats (2, 3) 112 / 120 us vs
-    // (1, 4) 127 / 118 (W6A8 at 512 tokens / W6A8-g128 at 301); down 75 / 65.5
-    // vs 68.7 / 63.8; INT8 90.6 + 64.2 vs 89.8 + 60.6 (197 tokens).
+    // pg_sub, pg_groups: 128-column blocks of a K step, workgroups per CU (3:
+    // 168 registers, 4: 128).  Measured for W6A8 gate/up at 512 tokens (2, 3)
+    // 112 us vs (1, 4) 127, down 75 vs 68.7; a W6A8-g128 layer at 301 tokens
+    // 207 vs 199; INT8 90.6 + 64.2 vs 89.8 + 60.6 (197 tokens).
     static constexpr int kSub = pg_sub(MODE, GATEUP);
     using Acc = std::conditional_t<kFp8, v4f, v4i>;
 };
@@ -187,7 +187,7 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
                 for (int c = 0; c < 2; ++c) {
                     if constexpr (MODE == 3) decode_w4a8_tab(raw[b][c].v, s.tab, w[c]);
                     else decode_wrow<MODE, false>(raw[b][c].v, n[c], nullptr, w[c]);
-                    load_b(next, b, c);
+                    if constexpr (MODE != 1) load_b(next, b, c);
                 }
 #pragma unroll
                 for (int mi = 0; mi < MT; ++mi) {
@@ -198,11 +198,24 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
                         acc[mi][c] = mfma_i8(a1, w[c].r[1], acc[mi][c]);
                     }
                 }
+                // INT8 products read the loaded registers themselves, so these
+                // are reloaded after them (before them the loop copied every
+                // block and waited for it: a layer at 197 tokens 186 -> 179 us;
+                // two or three steps ahead, at 3 workgroups per CU: 192).
+                if constexpr (MODE == 1) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) load_b(next, b, c);
+                }
             } else {
                 const v4f zero = {0, 0, 0, 0};
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    const float sw = f16_to_f32((uint16_t)raw[b][c].scale);
+                    // Converted here, not in the multiply-adds below: the loaded
+                    // word would stay live past the reload, which then takes
+                    // another register and a wait and a copy at the loop's end.
+                    float sw = f16_to_f32((uint16_t)raw[b][c].scale);
+                    asm volatile("" : "+v"(sw));
                     v8i lo, hi;
                     if (c > 0) __builtin_amdgcn_sched_barrier(0);
                     expand_w<F::kWf>(raw[b][c].v, lo, hi);
