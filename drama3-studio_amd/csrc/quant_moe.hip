@@ -477,6 +477,7 @@ __device__ __forceinline__ void group_pairs(int e, int lane, SmallGroups& g) {
 // rotation, so the two overlap.  Output: act = bf16(bf16(silu(g)) * u).
 constexpr int kQgUnits = 4;  // rotated 256-blocks per wave, 16 lanes each: rows * H / 256 <= 32
 
+template <int MODE>
 struct QGateUpLds {
     SmallGroups g;
     union {
@@ -488,9 +489,9 @@ struct QGateUpLds {
     float book[16];
     int rid[kSmallPairs];               // routed in the kernel: expert of each pair
     float rw[kSmallPairs];              // and its route weight (w_dtype-rounded, as stored)
-    alignas(16) int8_t qtab[256 * 16];  // mode 3: INT8 weight of (scale byte, code)
+    alignas(16) int8_t qtab[MODE == 3 ? 256 * 16 : 16];  // mode 3: INT8 weight of (scale byte, code)
     union {
-        float tb[kQWaves][kRotWaveDwords];  // rotation transposes
+        float tb[MODE != 0 ? kQWaves : 1][kRotWaveDwords];  // rotation transposes
         float red[kQWaves][kWave][12];      // cross-wave reduction (gate, up, third tile)
     };
 };
@@ -502,8 +503,10 @@ struct QGateUpLds {
 // The workgroup body, for work item (ai = active index, cg = column group);
 // each activation value h of pair p, column c goes to sink(p * I + c, bf16
 // bits of h).  A workgroup whose ai is past the active experts returns early.
-template <int MODE, int XT, int KBW, int NT, class Sink, class Pre>
-__device__ __forceinline__ void quant_gateup_body(const QuantGateUpArgs& a, QGateUpLds& s, int wai, int cg,
+// LAZY: weight rows stay as loaded until their products (the registers of the
+// decoded operands would hold the workgroups of a CU to two).
+template <int MODE, int XT, int KBW, int NT, bool LAZY, class Sink, class Pre>
+__device__ __forceinline__ void quant_gateup_body(const QuantGateUpArgs& a, QGateUpLds<MODE>& s, int wai, int cg,
                                                   Sink&& sink, Pre&& before_publish) {
     constexpr bool F16 = XT == kF16;
     constexpr int NX = NT == 3 ? KBW : 1;  // third-tile registers
@@ -658,19 +661,20 @@ __device__ __forceinline__ void quant_gateup_body(const QuantGateUpArgs& a, QGat
     }
     lds_barrier();
 
-    PackedRow bg[KBW], bu[KBW], bx[NX];
+    auto decode = [&](const PackedRaw& raw, int n, PackedRow& out) {
+        if constexpr (MODE == 3) decode_w4a8_tab(raw, s.qtab, out);  // one table for the workgroup's expert
+        else decode_wrow<MODE, F16>(raw, n, s.book, out);
+    };
+    constexpr int NB = LAZY ? 1 : KBW, NBX = LAZY ? 1 : NX;
+    PackedRow bg[NB], bu[NB], bx[NBX];
+    if constexpr (!LAZY) {
 #pragma unroll
-    for (int i = 0; i < KBW; ++i) {
-        const int kb = wave + i * kQWaves;
-        if (kb < KB) {
-            if constexpr (MODE == 3) {  // one table for the workgroup's expert
-                decode_w4a8_tab(rg[i], s.qtab, bg[i]);
-                decode_w4a8_tab(ru[i], s.qtab, bu[i]);
-                if constexpr (NT == 3) decode_w4a8_tab(rx[i], s.qtab, bx[i]);
-            } else {
-                decode_wrow<MODE, F16>(rg[i], ng, s.book, bg[i]);
-                decode_wrow<MODE, F16>(ru[i], nu, s.book, bu[i]);
-                if constexpr (NT == 3) decode_wrow<MODE, F16>(rx[i], nx, s.book, bx[i]);
+        for (int i = 0; i < KBW; ++i) {
+            const int kb = wave + i * kQWaves;
+            if (kb < KB) {
+                decode(rg[i], ng, bg[i]);
+                decode(ru[i], nu, bu[i]);
+                if constexpr (NT == 3) decode(rx[i], nx, bx[i]);
             }
         }
     }
@@ -686,39 +690,39 @@ __device__ __forceinline__ void quant_gateup_body(const QuantGateUpArgs& a, QGat
         for (int i = 0; i < KBW; ++i) {
             const int kb = wave + i * kQWaves;
             if (kb >= KB) continue;
-            if constexpr (MODE == 0) {
-                const uint16_t* xp = s.x.h + xr * H + kb * 128 + grp * 32;
+            constexpr int kT = MODE == 0 ? 4 : 2;  // 16-byte A operands of a block
+            const char* xp = MODE == 0 ? (const char*)(s.x.h + xr * H + kb * 128 + grp * 32)
+                                       : (const char*)(s.x.q + xr * H + kb * 128 + grp * 32);
+            v4i av[kT];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const v4i av = live ? *(const v4i*)(xp + 8 * t) : v4i{0, 0, 0, 0};
-                    if constexpr (F16) {
-                        fg = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, av),
-                                                                     __builtin_bit_cast(v8h, bg[i].r[t]), fg, 0, 0, 0);
-                        fu = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, av),
-                                                                     __builtin_bit_cast(v8h, bu[i].r[t]), fu, 0, 0, 0);
-                        if constexpr (NT == 3)
-                            fx = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, av),
-                                                                         __builtin_bit_cast(v8h, bx[i].r[t]), fx, 0, 0, 0);
-                    } else {
-                        fg = mfma_bf16(__builtin_bit_cast(v8bf, av), __builtin_bit_cast(v8bf, bg[i].r[t]), fg);
-                        fu = mfma_bf16(__builtin_bit_cast(v8bf, av), __builtin_bit_cast(v8bf, bu[i].r[t]), fu);
-                        if constexpr (NT == 3)
-                            fx = mfma_bf16(__builtin_bit_cast(v8bf, av), __builtin_bit_cast(v8bf, bx[i].r[t]), fx);
-                    }
+            for (int t = 0; t < kT; ++t) av[t] = live ? *(const v4i*)(xp + 16 * t) : v4i{0, 0, 0, 0};
+            auto products = [&](const PackedRow& b, v4f& f, v4i& n) {
+#pragma unroll
+                for (int t = 0; t < kT; ++t) {
+                    if constexpr (MODE != 0) n = mfma_i8(av[t], b.r[t], n);
+                    else if constexpr (F16)
+                        f = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, av[t]),
+                                                                    __builtin_bit_cast(v8h, b.r[t]), f, 0, 0, 0);
+                    else f = mfma_bf16(__builtin_bit_cast(v8bf, av[t]), __builtin_bit_cast(v8bf, b.r[t]), f);
                 }
-            } else {
-                const int8_t* xp = s.x.q + xr * H + kb * 128 + grp * 32;
-                const v4i a0 = live ? *(const v4i*)xp : v4i{0, 0, 0, 0};
-                const v4i a1 = live ? *(const v4i*)(xp + 16) : v4i{0, 0, 0, 0};
-                ig = mfma_i8(a0, bg[i].r[0], ig);
-                ig = mfma_i8(a1, bg[i].r[1], ig);
-                iu = mfma_i8(a0, bu[i].r[0], iu);
-                iu = mfma_i8(a1, bu[i].r[1], iu);
-                if constexpr (NT == 3) {
-                    ix = mfma_i8(a0, bx[i].r[0], ix);
-                    ix = mfma_i8(a1, bx[i].r[1], ix);
+            };
+            auto tile = [&](const PackedRaw& raw, int n, const PackedRow& decoded, v4f& f, v4i& acc) {
+                if constexpr (LAZY) {
+                    PackedRow b;
+                    PackedRaw fresh = raw;
+                    // decoded in this pass: hoisted out of the pass loop, the
+                    // operands of every tile would be live (and spill)
+                    if constexpr (MODE != 1) asm volatile("" : "+v"(fresh.a));
+                    decode(fresh, n, b);
+                    products(b, f, acc);
+                    __builtin_amdgcn_sched_barrier(0);  // one tile's operands live at a time
+                } else {
+                    products(decoded, f, acc);
                 }
-            }
+            };
+            tile(rg[i], ng, bg[LAZY ? 0 : i], fg, ig);
+            tile(ru[i], nu, bu[LAZY ? 0 : i], fu, iu);
+            if constexpr (NT == 3) tile(rx[i], nx, bx[LAZY ? 0 : i], fx, ix);
         }
         // cross-wave reduction (exact in int32 for modes 1-3)
 #pragma unroll
@@ -788,10 +792,15 @@ __device__ __forceinline__ void quant_gateup_body(const QuantGateUpArgs& a, QGat
     }
 }
 
+// Up to 128 registers: two workgroups per CU at least, three where a format
+// needs 80 or fewer (bounded to 80, W4A16 and W6A8 spill: a W4A16 decode layer
+// at 3 tokens x top-8 46 us; up to 128 with the rows decoded ahead 45.6; up to
+// 128 and decoded at their products 35.2, both with the down kernel's waves
+// as below).
 template <int MODE, int XT, int KBW, int NT>
-__global__ __launch_bounds__(kQThreads) void quant_gateup_decode_kernel(QuantGateUpArgs a) {
-    __shared__ QGateUpLds s;
-    quant_gateup_body<MODE, XT, KBW, NT>(
+__global__ __launch_bounds__(kQThreads, KBW <= 2 ? 4 : 2) void quant_gateup_decode_kernel(QuantGateUpArgs a) {
+    __shared__ QGateUpLds<MODE> s;
+    quant_gateup_body<MODE, XT, KBW, NT, true>(
         a, s, blockIdx.x, blockIdx.y, [&](int64_t i, uint16_t bits) { a.act[i] = bits; }, [] {});
 }
 
@@ -864,8 +873,14 @@ void launch_quant_gateup_decode(const QuantGateUpArgs& a, hipStream_t stream) {
 // (y = int32 dot * row scale * channel scale, or the fp32 dot), then the
 // workgroup sums each token's valid pairs in router slot order -- what
 // projection(weighted) + the combine of quantized_kernels.py:217-260 give.
-constexpr int kQdWaves = 4, kQdThreads = kQdWaves * kWave;
-constexpr int kQdGroups = 3;  // rotation groups (4 blocks, 16 lanes each) per wave: pairs * I / 256 <= 48
+// Eight waves: most calls' expert pairs of a workgroup are in flight at once
+// (four waves and rows decoded ahead took three serial rounds of loads for 24
+// experts; 16 waves leave 128 registers and spill).
+constexpr int kQdWaves = 8, kQdThreads = kQdWaves * kWave;
+constexpr int kQdMaxUnits = 48;  // rotated 256-blocks of a call: pairs * I / 256
+// rotation groups (4 blocks, 16 lanes each) per wave, and the waves that hold any
+constexpr int qd_groups(int waves) { return (kQdMaxUnits / 4 + waves - 1) / waves; }
+constexpr int qd_rot_waves(int waves) { return waves < kQdMaxUnits / 4 ? waves : kQdMaxUnits / 4; }
 
 template <int QDW>
 struct QDownLdsT {
@@ -873,7 +888,7 @@ struct QDownLdsT {
     union {
         struct {
             alignas(16) int8_t q[kQdMaxRotRows * kQdMaxI];  // modes 1-3: rotated INT8 hidden rows
-            float tb[QDW][kRotWaveDwords];                  // and the rotation transposes
+            float tb[qd_rot_waves(QDW)][kRotWaveDwords];                  // and the rotation transposes
         };
         alignas(16) uint16_t h[kQdMaxBf16];  // mode 0: bf16 hidden rows
     } act;
@@ -933,7 +948,7 @@ __device__ __forceinline__ void fetch_down_batch(const QuantProjArgs& w, const S
 template <int MODE, int KB2, int QDW, bool FUSED, class Prep, class Hidden>
 __device__ __forceinline__ void quant_down_body(const QuantDownArgs& a, QDownLdsT<QDW>& s, int tile,
                                                 const SmallGroups& fg, Prep&& prep, Hidden&& hidden) {
-    constexpr int QDT = QDW * kWave;
+    constexpr int QDT = QDW * kWave, kQdGroups = qd_groups(QDW);
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int col = lane % 16, grp = lane / 16;
     const QuantProjArgs& w = a.w2;
@@ -989,13 +1004,23 @@ __device__ __forceinline__ void quant_down_body(const QuantDownArgs& a, QDownLds
     const int n = n0 + (col & 7);
     DownBatch<KB2> cur;
     auto fetch_batch = [&](int bi) { fetch_down_batch<MODE, KB2>(w, g, bi, n, cur); };
-    PackedRow b[KB2];
+    // FUSED: a batch is decoded whole ahead of its products (the first one
+    // while the hidden rows are polled); else block by block between them
+    constexpr bool kLazy = !FUSED;
+    PackedRow b[kLazy ? 1 : KB2];
+    auto decode_block = [&](int kb, PackedRow& out) {
+        PackedRaw raw = cur.raw[kb];
+        if constexpr (kLazy && MODE != 1) asm volatile("" : "+v"(raw.a));  // not hoisted out of the pass loop
+        decode_wrow<MODE, false>(raw, n, s.book[wave][col < 8 ? 0 : 1], out);
+    };
     auto decode_batch = [&]() {
         if constexpr (MODE == 3) {
             if (lane < 32) s.book[wave][lane / 16][lane % 16] = cur.bk;  // read back by this wave only
         }
+        if constexpr (!kLazy) {
 #pragma unroll
-        for (int kb = 0; kb < KB2; ++kb) decode_wrow<MODE, false>(cur.raw[kb], n, s.book[wave][col < 8 ? 0 : 1], b[kb]);
+            for (int kb = 0; kb < KB2; ++kb) decode_block(kb, b[kb]);
+        }
     };
     // FUSED: wave 0 published the workgroup's h words and its memory counter
     // holds their stores, so the batches go to waves 1.. (a wait for the rows
@@ -1171,13 +1196,16 @@ __device__ __forceinline__ void quant_down_body(const QuantDownArgs& a, QDownLds
 #pragma unroll
                     for (int t = 0; t < kT; ++t) av[(kb + 1) & 1][t] = *(const v4i*)(xr + (kb + 1) * kBlockBytes + 16 * t);
                 }
+                if constexpr (kLazy) decode_block(kb, b[0]);
+                const PackedRow& bk = b[kLazy ? 0 : kb];
 #pragma unroll
                 for (int t = 0; t < kT; ++t) {
                     if constexpr (MODE == 0)
-                        fa = mfma_bf16(__builtin_bit_cast(v8bf, av[kb & 1][t]), __builtin_bit_cast(v8bf, b[kb].r[t]), fa);
+                        fa = mfma_bf16(__builtin_bit_cast(v8bf, av[kb & 1][t]), __builtin_bit_cast(v8bf, bk.r[t]), fa);
                     else
-                        ia = mfma_i8(av[kb & 1][t], b[kb].r[t], ia);
+                        ia = mfma_i8(av[kb & 1][t], bk.r[t], ia);
                 }
+                if constexpr (kLazy) __builtin_amdgcn_sched_barrier(0);  // one block's operands live at a time
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -1229,7 +1257,7 @@ __global__ __launch_bounds__(kQdThreads) void quant_down_decode_kernel(QuantDown
 bool quant_down_decode_fits(int mode, int pairs, int H, int I) {
     if (pairs < 1 || pairs > kSmallPairs || I > kQdMaxI || I % 128 != 0 || H % 8 != 0) return false;
     if (mode == 0) return pairs * I <= kQdMaxBf16;
-    return I % 256 == 0 && pairs <= kQdMaxRotRows && pairs * (I / 256) <= kQdWaves * kQdGroups * 4;
+    return I % 256 == 0 && pairs <= kQdMaxRotRows && pairs * (I / 256) <= kQdMaxUnits;
 }
 
 void launch_quant_down_decode(const QuantDownArgs& a, hipStream_t stream) {
@@ -1255,7 +1283,7 @@ void launch_quant_down_decode(const QuantDownArgs& a, hipStream_t stream) {
 
 template <int MODE, int XT, int KBW, int NT, int KB2>
 __global__ __launch_bounds__(kQThreads, 1) void quant_fused_decode_kernel(QuantFusedArgs a) {
-    __shared__ QGateUpLds su;
+    __shared__ QGateUpLds<MODE> su;
     __shared__ QDownLdsT<kQWaves> sd;
     __shared__ uint32_t s_epoch;
     const int B = blockIdx.x, G = gridDim.x, tid = threadIdx.x;
@@ -1274,7 +1302,7 @@ __global__ __launch_bounds__(kQThreads, 1) void quant_fused_decode_kernel(QuantF
         uint32_t* hbuf = nullptr;
         // wave 0 publishes after the body's reduction barrier, so the epoch
         // written just before the pass loop is in LDS by then
-        quant_gateup_body<MODE, XT, KBW, NT>(
+        quant_gateup_body<MODE, XT, KBW, NT, false>(
             a.up, su, B % min(a.up.pairs, a.up.experts), B / min(a.up.pairs, a.up.experts),
             [&](int64_t i, uint16_t bits) {
                 if (hbuf == nullptr) hbuf = a.ht + (int64_t)(s_epoch & 1) * kHandoffWords;
@@ -1283,7 +1311,7 @@ __global__ __launch_bounds__(kQThreads, 1) void quant_fused_decode_kernel(QuantF
             set_epoch);
     } else {
         // no gate/up item: route and group like the others
-        quant_gateup_body<MODE, XT, KBW, NT>(a.up, su, min(a.up.pairs, a.up.experts), 0,
+        quant_gateup_body<MODE, XT, KBW, NT, false>(a.up, su, min(a.up.pairs, a.up.experts), 0,
                                              [&](int64_t, uint16_t) {}, set_epoch);
     }
     // down: the route weights, the epoch (the ticket thread's wave alone waits

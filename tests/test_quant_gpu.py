@@ -213,6 +213,34 @@ def test_small_call_wide_gateup_workgroups(cuda, small_launches, mode, inter, to
     assert rel_inf(outs[True].float().cpu().numpy(), expected) < TOL
 
 
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("hidden,inter,tokens", [(2048, 768, 2), (2048, 768, 3), (2304, 1024, 2)])
+def test_small_call_repeated_experts(cuda, small_launches, mode, hidden, inter, tokens):
+    """All pairs on two experts: more than 16 (gate/up) and 8 (down) pairs of
+    one expert take several passes over the weight rows a wave holds as
+    loaded; (2304: 18 K blocks, a partly filled last round of the waves).
+    Bit-identical to the separate launches for modes 1-3."""
+    print_case("quant repeated experts", mode, hidden, inter, tokens)
+    g = torch.Generator().manual_seed(2600 + 16 * mode + tokens)
+    store = random_quantized_bank(mode, 4, hidden, inter, generator=g)
+    dev = to_device(store, cuda)
+    x = torch.randn(tokens, hidden, generator=g).bfloat16()
+    ids = torch.full((tokens, 8), 3, dtype=torch.int32)
+    ids[0, 0] = 1
+    weights = torch.softmax(torch.randn(tokens, 8, generator=g), -1).bfloat16()
+    backend = quantized.QuantizedExpertBackend(mode)
+    outs = {}
+    for single in (True, False):
+        small_launches(single)
+        outs[single] = backend.forward(x.to(cuda), ids.to(cuda), weights.to(cuda), dev)
+    if mode:
+        assert torch.equal(outs[True], outs[False])
+    else:
+        assert rel_inf(outs[True].float().cpu().numpy(), outs[False].float().cpu().numpy()) < TOL
+    expected = oracle_layer(store, x.float().numpy(), ids.numpy(), weights.float().numpy())
+    assert rel_inf(outs[True].float().cpu().numpy(), expected) < TOL
+
+
 def test_w4a16_asymmetric_zero_points(cuda):
     print_case("w4a16 asym")
     g = torch.Generator().manual_seed(404)
