@@ -561,20 +561,15 @@ void check_quant_rows(const void* x, int x_dtype, int64_t x_row_stride, int rows
 // W4A16 GEMM where its tile shape fits, else the column-group kernel.
 void launch_projection(const dmoe::QuantProjArgs& q, const QuantWorkspace& ws, int experts, int pairs,
                        hipStream_t stream) {
-    const int max_active = std::min(pairs, experts);
-    if (dmoe::packed_grouped_fits(q.mode, q.N, q.K, q.w_sn, q.s_sn)) {
-        dmoe::PackedGroupedArgs a{};
-        a.p = q;
-        a.tile_expert = ws.tile_expert;
-        a.tile_m0 = ws.tile_m0;
-        a.tile_count = ws.tile_count;
-        a.max_tiles = std::min(pairs, dmoe::max_block_tiles(pairs, experts, dmoe::kGroupM));
-        dmoe::launch_packed_grouped(a, stream);
-    } else if (dmoe::w4a16_grouped_fits(q)) {
-        dmoe::launch_w4a16_grouped(q, max_active, stream, pairs);
-    } else {
-        dmoe::launch_quant_projection(q, max_active, stream);
-    }
+    dmoe::PackedGroupedArgs a{};
+    a.p = q;
+    a.tile_expert = ws.tile_expert;
+    a.tile_m0 = ws.tile_m0;
+    a.tile_count = ws.tile_count;
+    a.max_tiles = std::min(pairs, dmoe::max_block_tiles(pairs, experts, dmoe::kGroupM));
+    if (dmoe::packed_grouped_fits(q.mode, q.N, q.K, q.w_sn, q.s_sn)) dmoe::launch_packed_grouped(a, stream);
+    else if (dmoe::w4a16_grouped_fits(q)) dmoe::launch_w4a16_grouped(a, stream);
+    else dmoe::launch_quant_projection(q, std::min(pairs, experts), stream);
 }
 
 // Permutation with the active-expert list (the grouping of every packed call).
@@ -1215,7 +1210,9 @@ int dmoe_w4a16_linear(const void* x, int x_dtype, int64_t x_row_stride, int rows
         q.out = out;
         q.out_row_stride = out_row_stride;
         q.dense_rows = rows;
-        dmoe::launch_w4a16_grouped(q, 1, as_stream(stream), rows);
+        dmoe::PackedGroupedArgs a{};
+        a.p = q;
+        dmoe::launch_w4a16_grouped(a, as_stream(stream));
     });
 }
 

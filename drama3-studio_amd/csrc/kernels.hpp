@@ -368,7 +368,6 @@ void launch_block_post(const BlockPostArgs& a, int cus, hipStream_t stream);
 // Tiled grouped W4A16 projection (w4a16_grouped.hip): mode 0 with gate/up
 // I % 64 == 0, or plain N % 128 == 0.
 bool w4a16_grouped_fits(const QuantProjArgs& a);
-void launch_w4a16_grouped(const QuantProjArgs& a, int max_active, hipStream_t stream, int pairs);
 
 // Tiled grouped projection of modes 1-5 (packed_grouped.hip) over 64-row tiles
 // (kGroupM).  p.order / p.offsets are the permutation, p.active is unused;
@@ -387,6 +386,8 @@ struct PackedGroupedArgs {
 };
 bool packed_grouped_fits(int mode, int N, int K, int64_t w_sn, int64_t s_sn);  // byte strides of a row
 void launch_packed_grouped(const PackedGroupedArgs& a, hipStream_t stream);
+// W4A16 (mode 0); a dense layer (p.dense_rows > 0) reads no tile map
+void launch_w4a16_grouped(const PackedGroupedArgs& a, hipStream_t stream);
 
 // Small packed calls (at most 64 route pairs): two launches that group the
 // pairs themselves from the route ids (no permutation launch).

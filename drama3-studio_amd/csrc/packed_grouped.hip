@@ -121,7 +121,8 @@ __device__ __forceinline__ BlockRaw<MODE> fetch_block(const RowBase& rb, uint32_
 
 // The tile (m0, mc rows of expert e) x 256 weight rows, MT 16-row units of it.
 template <int MODE, bool GATEUP, int MT>
-__device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLds<MODE, GATEUP>& s, int e, int m0, int mc) {
+__device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLds<MODE, GATEUP>& s, int e, int m0, int mc,
+                                            int ct) {
     using F = Fmt<MODE, GATEUP>;
     constexpr int kSub = F::kSub;
     const QuantProjArgs& p = a.p;
@@ -129,7 +130,7 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
     const int col = lane % 16, grp = lane / 16;
     const int half = p.N / 2, KB = p.K / 128, steps = KB / kSub;
     // this lane's two weight rows (rows past the matrix repeat its last; not stored)
-    const int n0 = GATEUP ? blockIdx.y * (kPgWaves * 16) + wave * 16 + col : blockIdx.y * (kPgWaves * 32) + wave * 32 + col;
+    const int n0 = GATEUP ? ct * (kPgWaves * 16) + wave * 16 + col : ct * (kPgWaves * 32) + wave * 32 + col;
     int n[2];
     n[0] = min(n0, (GATEUP ? half : p.N) - 1);
     n[1] = GATEUP ? half + n[0] : min(n0 + 16, p.N - 1);
@@ -316,18 +317,29 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
     }
 }
 
+// Column tiles of N weight rows.
+template <bool GATEUP>
+__host__ __device__ constexpr int pg_cols(int N) {
+    constexpr int kCols = kPgWaves * (GATEUP ? 16 : 32);
+    return ((GATEUP ? N / 2 : N) + kCols - 1) / kCols;
+}
+
 template <int MODE, bool GATEUP>
 __global__ __launch_bounds__(kPgThreads, pg_groups(MODE, GATEUP)) void packed_grouped_kernel(PackedGroupedArgs a) {
     __shared__ PackedLds<MODE, GATEUP> s;
-    const int tile = blockIdx.x;
-    if (tile >= *a.tile_count) return;
+    // tiles in multiples of the 8 XCDs inside a column tile: the column tiles
+    // of a row tile share its XCD's L2; what the grid holds beyond the call's
+    // tiles comes last and exits while the others finish
+    const int count = *a.tile_count, t8 = max((count + 7) / 8 * 8, 8);
+    const int tile = (int)blockIdx.x % t8, ct = (int)blockIdx.x / t8;
+    if (tile >= count || ct >= pg_cols<GATEUP>(a.p.N)) return;
     const int e = __builtin_amdgcn_readfirstlane(a.tile_expert[tile]);
     const int m0 = __builtin_amdgcn_readfirstlane(a.tile_m0[tile]);
     const int mc = min(kGroupM, a.p.offsets[e + 1] - m0);
-    if (mc <= 16) packed_tile<MODE, GATEUP, 1>(a, s, e, m0, mc);
-    else if (mc <= 32) packed_tile<MODE, GATEUP, 2>(a, s, e, m0, mc);
-    else if (mc <= 48) packed_tile<MODE, GATEUP, 3>(a, s, e, m0, mc);
-    else packed_tile<MODE, GATEUP, 4>(a, s, e, m0, mc);
+    if (mc <= 16) packed_tile<MODE, GATEUP, 1>(a, s, e, m0, mc, ct);
+    else if (mc <= 32) packed_tile<MODE, GATEUP, 2>(a, s, e, m0, mc, ct);
+    else if (mc <= 48) packed_tile<MODE, GATEUP, 3>(a, s, e, m0, mc, ct);
+    else packed_tile<MODE, GATEUP, 4>(a, s, e, m0, mc, ct);
 }
 
 }  // namespace
@@ -340,10 +352,7 @@ bool packed_grouped_fits(int mode, int N, int K, int64_t w_sn, int64_t s_sn) {
 
 template <int MODE, bool GATEUP>
 static void launch_mode(const PackedGroupedArgs& a, hipStream_t stream) {
-    constexpr int kCols = kPgWaves * (GATEUP ? 16 : 32);
-    const int cols = ((GATEUP ? a.p.N / 2 : a.p.N) + kCols - 1) / kCols;
-    // a multiple of the 8 XCDs: the column tiles of a row tile share its XCD's L2
-    const dim3 grid((unsigned)((a.max_tiles + 7) / 8 * 8), (unsigned)cols);
+    const dim3 grid((unsigned)((a.max_tiles + 7) / 8 * 8) * (unsigned)pg_cols<GATEUP>(a.p.N));
     hipLaunchKernelGGL((packed_grouped_kernel<MODE, GATEUP>), grid, dim3(kPgThreads), 0, stream, a);
 }
 
