@@ -37,7 +37,7 @@ namespace dmoe {
 
 namespace {
 
-constexpr int kUpWaves = 8, kUpThreads = kUpWaves * kWave;
+constexpr int kUpWaves = kDecodeUpWaves, kUpThreads = kUpWaves * kWave;
 // Down kernel waves per workgroup: each wave walks its own batches of two
 // experts, whose pair lists, activation rows and hidden scales are dependent
 // global reads; more waves split that chain. Eight where the kernel fits 256

@@ -26,6 +26,10 @@ constexpr int kGroupM = 64;
 constexpr int kFusedMaxPairs = 64;
 constexpr int kFusedMaxI = 1024;
 
+// Gate/up sums along K of the FP8 decode kernels: wave w of this many sums the
+// 128-column blocks w, w + 8, .. as one chain, and the chains add in wave order.
+constexpr int kDecodeUpWaves = 8;
+
 // Weight formats of the FP8-MFMA kernels (wfmt.hpp): E4M3 bytes, or 4- / 6-bit
 // integer codes with group-128 fp16 scales.
 enum { kWfFp8 = 0, kWfInt4 = 1, kWfInt6 = 2 };

@@ -8,8 +8,10 @@
 //   modes 4-5: FP8 rows x integer levels exact in E4M3 (wfmt.hpp), per
 //              128-column block acc = fma(dot * s_x, s_w, acc); gate/up rounded
 //              through the compute dtype, h = silu(gate) * up, FP8 per
-//              128-group; down: * route weight (fp32).  In gate/up s_x is
-//              constant along K and multiplies the sum once.
+//              128-group; down: * route weight (fp32).  Gate/up sums as the
+//              decode kernel's waves do (kDecodeUpWaves chains, added in
+//              order), so a route row's value does not depend on how its call
+//              was split: bit for bit that of a decode call.
 // Replaces the reference's Triton _quant_gemm over large batches
 // (src/drama_low_vram/quantized_kernels.py:115-214).
 //
@@ -48,7 +50,7 @@ constexpr int kPgWaves = 4, kPgThreads = kPgWaves * kWave;
 constexpr int kPgMaxHiddenBlocks = kMaxInter / 128;
 
 constexpr int pg_sub(int mode, bool gateup) { return (mode == 2 || mode == 3) && gateup ? 2 : 1; }
-constexpr int pg_groups(int mode, bool gateup) { return pg_sub(mode, gateup) == 2 ? 3 : 4; }
+constexpr int pg_groups(int mode, bool gateup) { return gateup && mode >= 2 ? 3 : 4; }
 
 template <int MODE, bool GATEUP>
 struct Fmt {
@@ -56,9 +58,18 @@ struct Fmt {
     static constexpr int kWf = MODE == 4 ? kWfInt4 : kWfInt6;
     // pg_sub, pg_groups: 128-column blocks of a K step, workgroups per CU (3:
     // 168 registers, 4: 128).  Measured for W6A8 gate/up at 512 tokens (2, 3)
-    // 112 us vs (1, 4) 127, down 75 vs 68.7; a W6A8-g128 layer at 301 tokens
-    // 207 vs 199; INT8 90.6 + 64.2 vs 89.8 + 60.6 (197 tokens).
+    // 112 us vs (1, 4) 127, down 75 vs 68.7; INT8 90.6 + 64.2 vs 89.8 + 60.6
+    // (197 tokens).
     static constexpr int kSub = pg_sub(MODE, GATEUP);
+    // Sums along K of the group-128 gate/up: the decode kernel's waves each sum
+    // a chain of K blocks and add the chains in wave order.  Two sums a result
+    // need 3 workgroups' registers (at 4 they spill: a W6A8-g128 layer at 301
+    // tokens 277 us), and the strided K order costs W6A8 its cache lines: the
+    // pieces of a line of high parts lie eight steps apart, with two streams of
+    // both planes in use the lines overflow an XCD's L2 (TCC misses 3.7 -> 6.3 M
+    // a launch, layer 202 -> 218 us; one sum in K order at 4 workgroups: 199).
+    // W4A8-g128, one plane: 149 us at 600 tokens, uniform, either way.
+    static constexpr int kChains = kFp8 && GATEUP ? kDecodeUpWaves : 0;
     using Acc = std::conditional_t<kFp8, v4f, v4i>;
 };
 
@@ -170,9 +181,13 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
             for (int q = 0; q < kChunks; ++q) *(v4i*)&s.a[buf][b][aoff + q * kRowStep * 128] = areg[b][q];
     };
     auto load_b = [&](int st, int b, int c) { raw[b][c] = fetch_block<MODE>(rb, wo[c], wo[c] + high, so[c], st * kSub + b); };
-    typename F::Acc acc[MT][2];
+    // kChains: `part` is the running chain and acc the sum of the chains before it
+    constexpr int MP = F::kChains ? MT : 1;
+    typename F::Acc acc[MT][2], part[MP][2];
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi) acc[mi][0] = acc[mi][1] = typename F::Acc{0, 0, 0, 0};
+#pragma unroll
+    for (int mi = 0; mi < MP; ++mi) part[mi][0] = part[mi][1] = typename F::Acc{0, 0, 0, 0};
 
     // Multiply step st; a weight block's registers take the same block of step
     // `next` as soon as it is decoded.
@@ -225,15 +240,12 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
                     for (int mi = 0; mi < MT; ++mi) {
                         const v4i a0 = *(const v4i*)(at + mi * 16 * 128 + o0), a1 = *(const v4i*)(at + mi * 16 * 128 + o1);
                         const v8i av = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-                        v4f rs = {1.0f, 1.0f, 1.0f, 1.0f};
-                        if constexpr (!GATEUP) rs = *(const v4f*)&s.rs[st * kSub + b][16 * mi + 4 * grp];
+                        const v4f rs = *(const v4f*)(GATEUP ? &s.sa[16 * mi + 4 * grp] : &s.rs[GATEUP ? 0 : st * kSub + b][16 * mi + 4 * grp]);
                         v4f d = mfma_fp8(av, lo, zero);
                         if constexpr (MODE == 5) d = mfma_fp8(av, hi, d);
+                        v4f& sum = F::kChains ? part[F::kChains ? mi : 0][c] : acc[mi][c];
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float t = GATEUP ? d[i] : d[i] * rs[i];
-                            acc[mi][c][i] = fmaf(t, sw, acc[mi][c][i]);
-                        }
+                        for (int i = 0; i < 4; ++i) sum[i] = fmaf(d[i] * rs[i], sw, sum[i]);
                     }
                 }
             }
@@ -265,12 +277,28 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
     // The barrier makes this step's activation rows visible; the buffer staged
     // into was read before it.  The last step loads itself again: no branch
     // around the loads, so the waits stay counted and never drain them.
-    for (int st = 0, buf = 0; st < steps; ++st, buf ^= 1) {
-        const int next = min(st + 1, steps - 1);
+    for (int i = 0, st = 0, buf = 0; i < steps; ++i, buf ^= 1) {
+        // kChains: steps w, w + kChains, .. of one chain w after the other
+        const bool end = F::kChains == 0 || st + F::kChains >= steps;
+        const int after = F::kChains == 0 ? st + 1 : end ? st % (F::kChains ? F::kChains : 1) + 1 : st + F::kChains;
+        const int next = i + 1 < steps ? after : st;
         load_a(next);
         lds_barrier();
         compute(st, next, buf);
+        if constexpr (F::kChains > 0) {
+            if (end) {
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi) {
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        acc[mi][c] += part[mi][c];
+                        part[mi][c] = typename F::Acc{0, 0, 0, 0};
+                    }
+                }
+            }
+        }
         stage_a(buf ^ 1);
+        st = next;
     }
 
     // epilogue: a lane holds column `col` of each 16 x 16 result, rows 4 grp + i
@@ -287,11 +315,11 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
                 const int r = 16 * mi + 4 * grp + i, pr = s.pair[r];
                 if (pr < 0) continue;
                 float y[2];
-                const float sa = F::kFp8 && !GATEUP ? 1.0f : s.sa[r];
                 if constexpr (F::kFp8) {
-                    y[0] = acc[mi][0][i] * sa;
-                    y[1] = acc[mi][1][i] * sa;
+                    y[0] = acc[mi][0][i];
+                    y[1] = acc[mi][1][i];
                 } else {
+                    const float sa = s.sa[r];
                     y[0] = bf16_round((float)acc[mi][0][i] * sa * sb[0]);
                     y[1] = bf16_round((float)acc[mi][1][i] * sa * sb[1]);
                 }

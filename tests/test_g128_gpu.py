@@ -295,3 +295,64 @@ def test_g128_tiled_row_edges(cuda, mode, hidden, inter):
     expected = np.concatenate([orc.fp8_expert_pairs(b13, b2, x[r].float().numpy(), ids[r].numpy(), w[r].numpy(),
                                                     x_group=hidden) for r in keep])
     assert rel_inf(out.cpu().numpy()[keep], expected) < TOL
+
+
+@pytest.mark.parametrize("mode", [4, 5])
+@pytest.mark.parametrize("hidden,inter,dtype", [
+    (256, 512, torch.bfloat16),    # 2 blocks of 128 along K: fewer than the decode kernel's 8 chains
+    (1408, 256, torch.float16),    # 11 blocks: chains of two and of one
+    (2048, 768, torch.bfloat16),   # every chain of two
+])
+def test_g128_large_calls_give_the_bits_of_small_ones(cuda, mode, hidden, inter, dtype):
+    """A route row's value does not depend on how its call is split: calls of
+    more than 256 pairs (the tiled GEMMs) equal the same rows in decode calls
+    bit for bit, as per-pair contributions, as layer sums and routed; and they
+    equal themselves with a workspace that holds decode calls only (the
+    consecutive decode calls of the same entry point)."""
+    import ctypes
+
+    from drama_moe.quantized import bank_struct
+
+    print_case("g128 large vs small calls", mode, hidden, inter)
+    experts, top_k, tokens = 12, 5, 70
+    store = bank_on(cuda, mode, experts, hidden, inter, 300 + mode + hidden)
+    g = torch.Generator().manual_seed(mode + hidden)
+    x = torch.randn(tokens, hidden, generator=g).to(dtype).to(cuda)
+    logits = (torch.randn(tokens, experts, generator=g) * 2).to(cuda)
+    backend = QuantizedExpertBackend(mode)
+    backend.status(cuda)
+    out, w, ids = backend.forward_routed(x, logits, top_k, store)
+    parts = [backend.forward_routed(x[t:t + 12], logits[t:t + 12], top_k, store) for t in range(0, tokens, 12)]
+    for k, whole in enumerate((out, w, ids)):
+        assert torch.equal(whole, torch.cat([p[k] for p in parts])), k
+    assert torch.equal(backend.forward(x, ids, w, store), out)
+
+    rows, flat, fw = x.repeat_interleave(top_k, 0), ids.reshape(-1, 1), w.reshape(-1, 1).float()
+    pairs = backend.forward_pairs(rows, flat, fw, store)
+    split = [backend.forward_pairs(rows[p:p + 64], flat[p:p + 64], fw[p:p + 64], store)
+             for p in range(0, len(rows), 64)]
+    assert torch.equal(pairs, torch.cat(split))
+
+    lib, bank = _lib.library(), bank_struct(store)
+    small = lib.dmoe_quant_workspace_bytes(ctypes.byref(bank), 256, 256)
+    assert small < lib.dmoe_quant_workspace_bytes(ctypes.byref(bank), tokens, tokens * top_k)
+    ws = torch.zeros(small, dtype=torch.uint8, device=cuda)
+    status = torch.zeros(1, dtype=torch.int32, device=cuda)
+    xs, code, stream = (_lib.ptr(x), _lib.dtype_code(dtype), x.stride(0)), _lib.dtype_code(dtype), _lib.stream_handle(cuda)
+    got, gids, gw = torch.empty_like(out), torch.empty_like(ids), torch.empty_like(w)
+    _lib.check(lib.dmoe_quant_moe_layer(
+        ctypes.byref(bank), *xs, tokens, _lib.ptr(logits), logits.stride(0), top_k, 1, _lib.ptr(gids), _lib.ptr(gw), code,
+        _lib.ptr(got), code, got.stride(0), _lib.ptr(ws), small, _lib.ptr(status), stream))
+    assert torch.equal(got, out) and torch.equal(gids, ids) and torch.equal(gw, w)
+    got.zero_()
+    _lib.check(lib.dmoe_quant_moe_forward(
+        ctypes.byref(bank), *xs, tokens, top_k, _lib.ptr(ids), _lib.dtype_code(ids.dtype), _lib.ptr(w), code,
+        tokens * top_k, top_k, _lib.ptr(got), code, got.stride(0), None, _lib.ptr(ws), small, _lib.ptr(status), stream))
+    assert torch.equal(got, out)
+    each = torch.empty_like(pairs)
+    _lib.check(lib.dmoe_quant_moe_forward(
+        ctypes.byref(bank), _lib.ptr(rows), code, rows.stride(0), len(rows), 1, _lib.ptr(flat),
+        _lib.dtype_code(flat.dtype), _lib.ptr(fw), _lib.F32, len(rows), 1, None, _lib.F32, 0, _lib.ptr(each),
+        _lib.ptr(ws), small, _lib.ptr(status), stream))
+    assert torch.equal(each, pairs)
+    assert int(status.item()) == 0 and backend.status(cuda) == 0
