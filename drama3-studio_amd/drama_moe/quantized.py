@@ -15,7 +15,7 @@ from torch import Tensor
 
 from . import _lib
 from .formats import QuantizedStore
-from .offload import MAX_PAIRS, _device_of, device_state
+from .offload import DECODE_PAIRS, MAX_PAIRS, _device_of, device_state
 
 MODE_NAMES = ("W4A16-GPTQ", "INT8-ConvRot/BF16", "W6A8/BF16", "W4A8-Codebook/BF16", "W4A8-G128/FP8",
               "W6A8-G128/FP8")
@@ -71,6 +71,17 @@ def rotate_quantize(x: Tensor):
         _lib.ptr(x), _lib.dtype_code(x.dtype), x.stride(0), x.shape[0], x.shape[1], _lib.ptr(q), _lib.ptr(scale),
         _lib.stream_handle(x.device)))
     return q, scale
+
+
+def _bank_workspace(state, bank: QuantBank, rows: int, pairs: int) -> Tensor:
+    """The workspace of a call over ``pairs`` route pairs.  A group-128 call
+    also runs, slower and with the same results, in the workspace of one decode
+    call: inside a graph capture, where the workspace cannot grow, it takes
+    what there is."""
+    need = _lib.library().dmoe_quant_workspace_bytes(ctypes.byref(bank), rows, pairs)
+    if bank.mode in (4, 5) and state.workspace.numel() < need and torch.cuda.is_current_stream_capturing():
+        need = _lib.library().dmoe_quant_workspace_bytes(ctypes.byref(bank), rows, min(pairs, DECODE_PAIRS))
+    return state.workspace_for(need)
 
 
 def projection(x: Tensor, ids: Tensor, weights: Tensor, bank: Tensor, scales: Tensor, *, mode: int,
@@ -136,7 +147,7 @@ class QuantizedExpertBackend:
         lib = _lib.library()
         state = device_state(device)
         pairs = ids.numel()
-        ws = state.workspace_for(lib.dmoe_quant_workspace_bytes(ctypes.byref(bank), rows, pairs))
+        ws = _bank_workspace(state, bank, rows, pairs)
         _lib.check(lib.dmoe_quant_moe_forward(
             ctypes.byref(bank), _lib.ptr(x), _lib.dtype_code(x.dtype), x.stride(0), rows, row_div,
             _lib.ptr(ids), _lib.dtype_code(ids.dtype), _lib.ptr(weights), _lib.dtype_code(weights.dtype), pairs,
@@ -199,7 +210,7 @@ class QuantizedExpertBackend:
         bank = bank_struct(staged)
         lib = _lib.library()
         state = device_state(device)
-        ws = state.workspace_for(lib.dmoe_quant_workspace_bytes(ctypes.byref(bank), tokens, tokens * top_k))
+        ws = _bank_workspace(state, bank, tokens, tokens * top_k)
         _lib.check(lib.dmoe_quant_moe_layer(
             ctypes.byref(bank), _lib.ptr(x), _lib.dtype_code(x.dtype), x.stride(0), tokens, _lib.ptr(logits),
             logits.stride(0), top_k, int(renormalize), _lib.ptr(ids), _lib.ptr(weights),

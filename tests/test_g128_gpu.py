@@ -356,3 +356,39 @@ def test_g128_large_calls_give_the_bits_of_small_ones(cuda, mode, hidden, inter,
         _lib.ptr(ws), small, _lib.ptr(status), stream))
     assert torch.equal(each, pairs)
     assert int(status.item()) == 0 and backend.status(cuda) == 0
+
+
+@pytest.mark.parametrize("mode", [4, 5])
+def test_g128_capture_of_a_larger_call_than_the_warm_one(cuda, mode, monkeypatch):
+    """The workspace of a 256-pair call is enough to capture a 560-pair one:
+    it runs as decode calls then, with the eager call's results."""
+    from drama_moe import offload
+
+    print_case("g128 capture beyond the warm call", mode)
+    store = bank_on(cuda, mode, 16, 512, 256, 400 + mode)
+    g = torch.Generator().manual_seed(40 + mode)
+    x = torch.randn(70, 512, generator=g).bfloat16().to(cuda)
+    logits = torch.randn(70, 16, generator=g).to(cuda)
+    backend = QuantizedExpertBackend(mode)
+    want, w, ids = backend.forward_routed(x, logits, 8, store)
+    torch.cuda.synchronize()
+    state = offload._DeviceState(want.device)
+    monkeypatch.setitem(offload._STATES, want.device, state)
+    backend.forward_routed(x[:32], logits[:32], 8, store)
+    torch.cuda.synchronize()
+    warm = state.workspace.numel()
+    stream = torch.cuda.Stream(cuda)
+    stream.wait_stream(torch.cuda.current_stream(cuda))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        routed = backend.forward_routed(x, logits, 8, store)
+        layer = backend.forward(x, ids, w, store)
+    assert state.workspace.numel() == warm
+    for replay in range(3):
+        for t in (*routed, layer):
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(routed[0], want) and torch.equal(routed[1], w) and torch.equal(routed[2], ids), replay
+        assert torch.equal(layer, want), replay
+    assert backend.status(cuda) == 0
