@@ -1,14 +1,14 @@
 """Arithmetic identities the packed-bank kernels rely on, checked exhaustively
 on the CPU.
 
-W6A8 dequantization (quant_moe.hip, decode_wrow for mode 2) turns a 6-bit code
-c and the E4M3 scale byte of its 16-code group into the INT8 weight
+W6A8 dequantization (packed_decode.hpp, decode_wrow for mode 2) turns a 6-bit
+code c and the E4M3 scale byte of its 16-code group into the INT8 weight
 q8(c - 32, rel) = clamp(rint((c - 32) * rel), -127, 127) (the reference's
 level * relative-scale rounding, quantized_kernels.py:148-173) in packed fp16
-arithmetic: x = fp16(1024 + c), v = (x - 1056) * rel, clamped to [-127, 127],
-then + 1536, whose low byte is the INT8 value.  numpy's float16 operations
-round exactly as the hardware's (the exact results fit float32 before the one
-rounding to float16), so every (code, scale byte) pair is checked here.
+arithmetic: the half 0x5400 | c << 4 is 64 + c, v = fma(64 + c, rel, -96 rel),
+clamped to [-127, 127], then + 1536, whose low byte is the INT8 value.  The
+fma's exact value fits float64 before its one rounding to float16, so every
+(code, scale byte) pair is checked here as the hardware computes it.
 """
 import numpy as np
 import torch
@@ -21,9 +21,10 @@ def q8(level: np.float32, rel: np.float32) -> int:
     return int(min(max(np.rint(v), np.float32(-127)), np.float32(127)))
 
 
-def packed_fp16(code: int, rel: np.float32) -> int:
-    x = np.float16(1024 + code)
-    v = np.float16(np.float16(x - np.float16(1056)) * np.float16(rel))
+def packed_fp16(code: int, rel: np.float32, offset: int = 96) -> int:
+    x = np.array(0x5400 | code << 4, np.uint16).view(np.float16)
+    bias = np.float16(np.float64(np.float16(rel)) * -offset)
+    v = np.float16(np.float64(x) * np.float64(np.float16(rel)) + np.float64(bias))  # one rounding: fma
     v = np.float16(-127) if np.isnan(v) else max(v, np.float16(-127))  # maxNum
     v = min(v, np.float16(127))
     m = np.float16(v + np.float16(1536))
@@ -41,8 +42,7 @@ def test_w6_packed_fp16_dequant_equals_q8_for_every_code_and_scale_byte():
 
 
 def test_packed_fp16_check_catches_a_wrong_offset():
-    # the same sequence with 1055 in place of 1056 (level off by one) must fail
+    # 95 in place of 96 (level off by one) must fail
     rel = np.float32(torch.tensor([0x38], dtype=torch.uint8).view(torch.float8_e4m3fn).float().item())
-    x = np.float16(1024 + 40)
-    wrong = np.float16(np.float16(x - np.float16(1055)) * np.float16(rel))
-    assert int(np.rint(wrong)) != q8(np.float32(40 - 32), rel)
+    assert packed_fp16(40, rel) == q8(np.float32(40 - 32), rel)
+    assert packed_fp16(40, rel, offset=95) != q8(np.float32(40 - 32), rel)
