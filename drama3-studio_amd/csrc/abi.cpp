@@ -557,8 +557,15 @@ void check_quant_rows(const void* x, int x_dtype, int64_t x_row_stride, int rows
     require(row_div >= 1 && (int64_t)(pairs - 1) / row_div < rows, "pairs read past the activation rows");
 }
 
-// A grouped packed projection: the tiled 8-bit GEMM (modes 1-3), the tiled
-// W4A16 GEMM where its tile shape fits, else the column-group kernel.
+// The kernels of a call's grouped projections read the tile map (the tiled
+// ones) or the active-expert list (column-group).
+enum class Grouped { kPacked, kW4A16, kColumns };
+
+Grouped grouped_kind(const dmoe::QuantProjArgs& q) {
+    if (dmoe::packed_grouped_fits(q.mode, q.N, q.K, q.w_sn, q.s_sn)) return Grouped::kPacked;
+    return dmoe::w4a16_grouped_fits(q) ? Grouped::kW4A16 : Grouped::kColumns;
+}
+
 void launch_projection(const dmoe::QuantProjArgs& q, const QuantWorkspace& ws, int experts, int pairs,
                        hipStream_t stream) {
     dmoe::PackedGroupedArgs a{};
@@ -567,18 +574,21 @@ void launch_projection(const dmoe::QuantProjArgs& q, const QuantWorkspace& ws, i
     a.tile_m0 = ws.tile_m0;
     a.tile_count = ws.tile_count;
     a.max_tiles = std::min(pairs, dmoe::max_block_tiles(pairs, experts, dmoe::kGroupM));
-    if (dmoe::packed_grouped_fits(q.mode, q.N, q.K, q.w_sn, q.s_sn)) dmoe::launch_packed_grouped(a, stream);
-    else if (dmoe::w4a16_grouped_fits(q)) dmoe::launch_w4a16_grouped(a, stream);
-    else dmoe::launch_quant_projection(q, std::min(pairs, experts), stream);
+    a.experts = experts;
+    switch (grouped_kind(q)) {
+        case Grouped::kPacked: dmoe::launch_packed_grouped(a, stream); break;
+        case Grouped::kW4A16: dmoe::launch_w4a16_grouped(a, stream); break;
+        default: dmoe::launch_quant_projection(q, std::min(pairs, experts), stream);
+    }
 }
 
-// Permutation with the active-expert list (the grouping of every packed call).
-void quant_group(const void* ids, int ids_dtype, int pairs, int experts, const QuantWorkspace& ws, int* status,
-                 hipStream_t stream) {
+// Permutation of a call with the lists its projections read.
+void quant_group(const void* ids, int ids_dtype, int pairs, int experts, const QuantWorkspace& ws, bool tiles,
+                 bool list, int* status, hipStream_t stream) {
     dmoe::PermuteArgs pa{ids, ids_dtype, pairs, experts, ws.order, ws.counts, ws.offsets, status,
-                         ws.permute_scratch, ws.permute_scratch + pairs, ws.active, dmoe::kGroupM,
-                         dmoe::max_block_tiles(pairs, experts, dmoe::kGroupM), ws.tile_expert, ws.tile_m0,
-                         ws.tile_count};
+                         ws.permute_scratch, ws.permute_scratch + pairs, list ? ws.active : nullptr, dmoe::kGroupM,
+                         dmoe::max_block_tiles(pairs, experts, dmoe::kGroupM), tiles ? ws.tile_expert : nullptr,
+                         ws.tile_m0, ws.tile_count};
     dmoe::launch_permute(pa, stream);
 }
 
@@ -686,6 +696,7 @@ void g128_grouped_call(const BankGeom& g, const Activations& x, const dmoe::Rout
         a.tile_m0 = ws.tile_m0;
         a.tile_count = ws.tile_count;
         a.max_tiles = std::min(pairs, tiles);
+        a.experts = g.experts;
         a.gu_dtype = x.x_dtype;
         return a;
     };
@@ -1342,7 +1353,8 @@ int dmoe_quant_projection(const DmoeQuantProj* proj, int experts, int mode, cons
         require(out != nullptr && out_row_stride >= q.N, "output [pairs, N] is required");
         const QuantWorkspace ws = take_quant_workspace(rows, pairs, experts, q.K, 0, workspace, workspace_bytes);
         hipStream_t st = as_stream(stream);
-        quant_group(ids, ids_dtype, pairs, experts, ws, status, st);
+        const bool tiles = grouped_kind(q) != Grouped::kColumns;
+        quant_group(ids, ids_dtype, pairs, experts, ws, tiles, !tiles, status, st);
         quant_operand(q, x, x_dtype, x_row_stride, rows, q.K, ws.xq, ws.xs, st);
         q.row_div = row_div;
         q.order = ws.order;
@@ -1412,7 +1424,12 @@ static void quant_forward_impl(const DmoeQuantBank* bank, const void* x, int x_d
                                      route->renormalize != 0, route->ids_out, route->weights_out, route->w_dtype};
             dmoe::launch_route_topk(ra, st);
         }
-        if (!small_up || !small_dn) quant_group(ids, ids_dtype, pairs, E, ws, status, st);
+        up.gateup = 1;
+        const auto grouped = [&](bool tiled) {
+            return (!small_up && (grouped_kind(up) != Grouped::kColumns) == tiled) ||
+                   (!small_dn && (grouped_kind(dn) != Grouped::kColumns) == tiled);
+        };
+        if (!small_up || !small_dn) quant_group(ids, ids_dtype, pairs, E, ws, grouped(true), grouped(false), status, st);
 
         if (small_up) {
             dmoe::QuantGateUpArgs ga{up, x, x_dtype, x_row_stride, rows, row_div, ids, ids_dtype, E, pairs,
@@ -1432,7 +1449,6 @@ static void quant_forward_impl(const DmoeQuantBank* bank, const void* x, int x_d
             up.order = ws.order;
             up.offsets = ws.offsets;
             up.active = ws.active;
-            up.gateup = 1;
             up.act = ws.act;
             up.status = status;
             launch_projection(up, ws, E, pairs, st);

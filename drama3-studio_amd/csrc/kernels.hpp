@@ -379,6 +379,7 @@ struct PackedGroupedArgs {
     const int32_t* tile_m0;
     const int32_t* tile_count;
     int max_tiles;
+    int experts;
     // modes 4, 5
     int gu_dtype;           // type gate and up are rounded through
     float* h32;             // gate/up out: silu(gate) * up [sorted position, N / 2]

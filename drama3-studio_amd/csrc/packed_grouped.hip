@@ -38,6 +38,7 @@
 #include "fp8_util.hpp"
 #include "kernels.hpp"
 #include "packed_decode.hpp"
+#include "tile_map.hpp"
 
 namespace dmoe {
 
@@ -355,15 +356,9 @@ __host__ __device__ constexpr int pg_cols(int N) {
 template <int MODE, bool GATEUP>
 __global__ __launch_bounds__(kPgThreads, pg_groups(MODE, GATEUP)) void packed_grouped_kernel(PackedGroupedArgs a) {
     __shared__ PackedLds<MODE, GATEUP> s;
-    // tiles in multiples of the 8 XCDs inside a column tile: the column tiles
-    // of a row tile share its XCD's L2; what the grid holds beyond the call's
-    // tiles comes last and exits while the others finish
-    const int count = *a.tile_count, t8 = max((count + 7) / 8 * 8, 8);
-    const int tile = (int)blockIdx.x % t8, ct = (int)blockIdx.x / t8;
-    if (tile >= count || ct >= pg_cols<GATEUP>(a.p.N)) return;
-    const int e = __builtin_amdgcn_readfirstlane(a.tile_expert[tile]);
-    const int m0 = __builtin_amdgcn_readfirstlane(a.tile_m0[tile]);
-    const int mc = min(kGroupM, a.p.offsets[e + 1] - m0);
+    TileWork t;
+    if (!take_tile(a, pg_cols<GATEUP>(a.p.N), t)) return;
+    const int e = __builtin_amdgcn_readfirstlane(t.e), m0 = __builtin_amdgcn_readfirstlane(t.m0), mc = t.mc, ct = t.ct;
     if (mc <= 16) packed_tile<MODE, GATEUP, 1>(a, s, e, m0, mc, ct);
     else if (mc <= 32) packed_tile<MODE, GATEUP, 2>(a, s, e, m0, mc, ct);
     else if (mc <= 48) packed_tile<MODE, GATEUP, 3>(a, s, e, m0, mc, ct);
@@ -380,7 +375,7 @@ bool packed_grouped_fits(int mode, int N, int K, int64_t w_sn, int64_t s_sn) {
 
 template <int MODE, bool GATEUP>
 static void launch_mode(const PackedGroupedArgs& a, hipStream_t stream) {
-    const dim3 grid((unsigned)((a.max_tiles + 7) / 8 * 8) * (unsigned)pg_cols<GATEUP>(a.p.N));
+    const dim3 grid(tile_grid(a.max_tiles, pg_cols<GATEUP>(a.p.N)));
     hipLaunchKernelGGL((packed_grouped_kernel<MODE, GATEUP>), grid, dim3(kPgThreads), 0, stream, a);
 }
 

@@ -14,8 +14,13 @@
 // down tiles 128 output rows.  Each wave owns two 16-column MFMA tiles.  (A
 // workgroup per expert streaming its tiles, as many of them at once as the
 // average expert has, left the chip waiting for the popular experts: a layer
-// at 600 tokens, Zipf(1.1) routing, 578 us against 194; at 512, uniform, 157 against 158.6.)  A dense layer's
-// rows stream through in 64-row chunks.  Per 128-column K block:
+// at 600 tokens, Zipf(1.1) routing, 576 us against 195; uniform, 512 tokens
+// 160 / 159, E 32 H 4096 I 1536 at 600 373 / 362; where K loops are short a
+// second tile in the same workgroup costs less than another one: E 16 H 512
+// I 256 at 1500 63 / 69.)  A workgroup's first loads go out as the tile map
+// names them, the rows' pair list and the weights together (rows before
+// weights: 512 tokens 162 us).  A dense layer's rows stream through in 64-row
+// chunks.  Per 128-column K block:
 //   * the chunk's 64 activation rows (16 KB) go global -> LDS with direct
 //     copies (gathered rows, no registers in between), double-buffered, the
 //     16-byte chunk c of row r stored at c ^ (r % 16) so the 16 rows an MFMA
@@ -34,6 +39,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "tile_map.hpp"
 
 namespace dmoe {
 
@@ -134,15 +140,12 @@ __global__ __launch_bounds__(kW4Threads) void w4a16_grouped_kernel(PackedGrouped
     const QuantProjArgs& a = args.p;
     int e = 0, pend = a.dense_rows, mbeg = (int)blockIdx.z * kW4Rows, ct = blockIdx.x;  // dense: chunks z, z + gridDim.z, ...
     if constexpr (!DENSE) {
-        // tiles in multiples of the 8 XCDs inside a column tile: the column
-        // tiles of a row tile share its XCD's L2; what the grid holds beyond
-        // the call's tiles comes last and exits while the others finish
-        const int t8 = max((*args.tile_count + 7) / 8 * 8, 8), tile = (int)blockIdx.x % t8;
-        ct = (int)blockIdx.x / t8;
-        if (ct >= a.N / 128 || tile >= *args.tile_count) return;
-        e = args.tile_expert[tile];
-        pend = a.offsets[e + 1];
-        mbeg = args.tile_m0[tile];
+        TileWork t;
+        if (!take_tile(args, a.N / 128, t)) return;
+        e = t.e;
+        ct = t.ct;
+        mbeg = t.m0;
+        pend = t.m0 + t.mc;
     }
     const int mend = DENSE ? pend : mbeg + 1;
     const int KB = a.K / 128, half = a.N / 2;
@@ -173,15 +176,20 @@ __global__ __launch_bounds__(kW4Threads) void w4a16_grouped_kernel(PackedGrouped
     auto a_off = [&](int mi, int t) { return (16 * mi + col) * 256 + (((4 * g + t) ^ col) * 16); };
 
     for (int m0 = mbeg; m0 < mend; m0 += (int)gridDim.z * kW4Rows) {
-        __syncthreads();  // the previous chunk is done with the row table and buffers
+        // the chunk's rows, then the first weights while they are on their way
+        const int pos = m0 + (int)threadIdx.x % kW4Rows, pc = pos < pend ? pos : m0;
+        const int p = DENSE ? pc : a.order[pc];
+        asm volatile("" ::: "memory");
+        W4Raw raw[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) raw[c] = w4_fetch(a, wrow[c], srow[c], zrow[c], 0, g);
+        asm volatile("" ::: "memory");
+        lds_barrier();  // the previous chunk is done with the row table and buffers
         if (threadIdx.x < kW4Rows) {
-            const int pos = m0 + (int)threadIdx.x;
-            const int pc = pos < pend ? pos : m0;
-            const int p = DENSE ? pc : a.order[pc];
             s.row[threadIdx.x] = p / a.row_div;
             s.pair[threadIdx.x] = pos < pend ? p : -1;
         }
-        __syncthreads();
+        lds_barrier();
         const uint16_t* xsrc[kW4ACopies];
 #pragma unroll
         for (int q = 0; q < kW4ACopies; ++q) {
@@ -197,10 +205,6 @@ __global__ __launch_bounds__(kW4Threads) void w4a16_grouped_kernel(PackedGrouped
         v4f acc[4][2];
 #pragma unroll
         for (int mi = 0; mi < 4; ++mi) acc[mi][0] = acc[mi][1] = v4f{0, 0, 0, 0};
-        W4Raw raw[2];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) raw[c] = w4_fetch(a, wrow[c], srow[c], zrow[c], 0, g);
-        asm volatile("" ::: "memory");
         issue_a(0, 0);
         asm volatile("" ::: "memory");
         for (int kb = 0; kb < KB; ++kb) {
@@ -272,7 +276,7 @@ void launch_w4a16_grouped(const PackedGroupedArgs& args, hipStream_t stream) {
     const QuantProjArgs& a = args.p;
     const unsigned cols = (unsigned)(a.N / 128);  // 64 gate + 64 up rows, or 128 output rows
     const int chunks = std::min(256, (a.dense_rows + kW4Rows - 1) / kW4Rows);
-    const dim3 tiles((unsigned)((args.max_tiles + 7) / 8 * 8) * cols), dense(cols, 1, (unsigned)chunks);
+    const dim3 tiles(tile_grid(args.max_tiles, (int)cols)), dense(cols, 1, (unsigned)chunks);
     auto go = [&](auto kernel, dim3 grid) { hipLaunchKernelGGL(kernel, grid, dim3(kW4Threads), 0, stream, args); };
     if (a.dense_rows > 0)
         a.x_f16 ? go(w4a16_grouped_kernel<false, true, true>, dense) : go(w4a16_grouped_kernel<false, false, true>, dense);

@@ -98,10 +98,15 @@ int main() {
                 for (int e : experts) {
                     if (H >= 4096 && p > 65536) continue;  // keep the sweep to sizes a call can have
                     check(run("prefill", [&](dmoe::Carver& c) { dmoe::prefill_layout(c, p, e, H, I); }));
+                    const Logged g128 = run("group-128 prefill", [&](dmoe::Carver& c) { dmoe::prefill_layout(c, p, e, H, I, true); });
+                    check(g128);
+                    const Region& partial = g128.regions.back();  // also the fp32 hidden rows
+                    if (std::strcmp(partial.name, "partials fp32") != 0 || partial.bytes < (size_t)p * (H > I ? H : I) * 4)
+                        fail("too small for the fp32 hidden rows", g128.layout, partial);
                     check(run("packed", [&](dmoe::Carver& c) { dmoe::quant_layout(c, (p + 7) / 8, p, e, H, I); }));
                     check(run("packed rows", [&](dmoe::Carver& c) { dmoe::quant_layout(c, p, p, e, H, I); }));
                     check(run("moe_align", [&](dmoe::Carver& c) { dmoe::align_layout(c, p, e, 16); }));
-                    layouts += 4;
+                    layouts += 5;
                 }
             for (int p : decode_pairs)
                 for (int e : experts) {

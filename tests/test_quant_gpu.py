@@ -401,25 +401,49 @@ def test_gptq_linear_matches_dequantize_then_matmul(cuda, rows, n, k, x_dtype):
 
 
 @pytest.mark.parametrize("mode", [1, 2, 3])
-@pytest.mark.parametrize("n,k,weighted", [(144, 256, True), (16, 1024, False)])
+@pytest.mark.parametrize("n,k,weighted", [
+    (1168, 256, True),    # enough workgroups for the tiled GEMM, N past its last whole column tile
+    (1296, 1024, False),  # an unweighted call, eight K blocks
+    (144, 256, True),     # too few: the column-group kernel (1-5 passes an expert)
+    (16, 1024, False),
+])
 def test_tiled_projection_row_and_column_edges(cuda, mode, n, k, weighted):
-    """The tiled 8-bit GEMM where its tiles end: experts of 1, 16, 17, 32, 33,
-    48, 49, 64, 65 and 0 rows, invalid ids, N past the last whole column tile
-    and below one.  INT32 sums and the two scale products are exact restatements
-    of the oracle's, so bf16 results differ by rounding ties only."""
+    """Both grouped kernels where their tiles and passes end: experts of 1, 16,
+    17, 32, 33, 48, 49, 64, 65 and 0 rows, invalid ids, N off the column tile.
+    INT32 sums and the two scale products are exact restatements of the
+    oracle's, so bf16 results differ by rounding ties only."""
     print_case("tiled projection edges", mode, n, k, weighted)
     g = torch.Generator().manual_seed(10 * mode + n)
     counts = [1, 16, 17, 32, 33, 0, 48, 49, 64, 65]
-    store = random_quantized_bank(mode, len(counts), k, max(256, n), generator=g)
+    store = random_quantized_bank(mode, len(counts), k, max(256, (n + 1) // 2), generator=g)
     bank, scales = store.w13_weight[:, :n], store.w13_scale_inv[:, :n]
-    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)] + [torch.tensor([-1, len(counts)])])
     ids = flat[torch.randperm(len(flat), generator=g)]
-    ids[3], ids[200] = -1, len(counts)
     x = torch.randn(len(ids), k, generator=g).bfloat16()
     w = torch.rand(len(ids), generator=g) + 0.1
     out = quantized.projection(x.to(cuda), ids.to(cuda), w.to(cuda), bank.to(cuda), scales.to(cuda), mode=mode,
                                weighted=weighted)
     keep = [r for r in range(len(ids)) if 0 <= int(ids[r]) < len(counts)]
+    assert torch.bincount(ids[keep], minlength=len(counts)).tolist() == counts
     b = orc.QuantBank(mode, bank.contiguous().numpy(), scales.contiguous().numpy(), n, k)
     expected = orc.quant_projection(b, x.float().numpy()[keep], ids.numpy()[keep], w.numpy()[keep], weighted=weighted)
     assert rel_inf(out.float().cpu().numpy()[keep], expected) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("mode", [1, 2, 3])
+@pytest.mark.parametrize("hidden,inter", [(256, 1280), (1280, 256)])
+def test_layer_with_one_tiled_and_one_column_group_projection(cuda, mode, hidden, inter):
+    """Gate/up tiled and down column-group, and the other way round: the
+    permutation writes the lists of both.  Experts of every tile edge."""
+    print_case("mixed grouped projections", mode, hidden, inter)
+    g = torch.Generator().manual_seed(mode * inter)
+    counts = [1, 16, 17, 32, 33, 0, 48, 49, 64, 65]
+    store = random_quantized_bank(mode, len(counts), hidden, inter, generator=g)
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    ids = flat[torch.randperm(len(flat), generator=g)][:, None]
+    x = torch.randn(len(ids), hidden, generator=g).bfloat16()
+    w = torch.rand(len(ids), 1, generator=g) + 0.1
+    backend = quantized.QuantizedExpertBackend(mode)
+    out = backend.forward_pairs(x.to(cuda), ids.to(cuda), w.to(cuda), to_device(store, cuda))
+    expected = oracle_layer(store, x.float().numpy(), ids.numpy(), w.numpy())
+    assert rel_inf(out.cpu().numpy(), expected) < TOL
