@@ -65,11 +65,7 @@ struct Fmt {
     // Sums along K of the group-128 gate/up: the decode kernel's waves each sum
     // a chain of K blocks and add the chains in wave order.  Two sums a result
     // need 3 workgroups' registers (at 4 they spill: a W6A8-g128 layer at 301
-    // tokens 277 us), and the strided K order costs W6A8 its cache lines: the
-    // pieces of a line of high parts lie eight steps apart, with two streams of
-    // both planes in use the lines overflow an XCD's L2 (TCC misses 3.7 -> 6.3 M
-    // a launch, layer 202 -> 218 us; one sum in K order at 4 workgroups: 199).
-    // W4A8-g128, one plane: 149 us at 600 tokens, uniform, either way.
+    // tokens 277 us).
     static constexpr int kChains = kFp8 && GATEUP ? kDecodeUpWaves : 0;
     using Acc = std::conditional_t<kFp8, v4f, v4i>;
 };
@@ -131,8 +127,16 @@ __device__ __forceinline__ BlockRaw<MODE> fetch_block(const RowBase& rb, uint32_
     return r;
 }
 
-// The tile (m0, mc rows of expert e) x 256 weight rows, MT 16-row units of it.
-template <int MODE, bool GATEUP, int MT>
+// The tile (m0, mc rows of expert e) x 128 weight rows, MT 16-row units of it.
+// OPEN (kChains): chains summed side by side; it divides the K blocks.  A chain's
+// blocks lie eight apart, so one chain at a time finds the pieces of a cache line
+// of W6A8-g128's high parts steps apart, and with two streams of both planes in
+// use the lines overflow an XCD's L2 (TCC misses of a launch 3.7 -> 6.3 M).  Open chains
+// visit neighbouring blocks; the registers hold 4 chains up to 32 rows, 2 up to
+// 48 and one above (2 above: 51 spills).  A layer at 40 / 128 / 600 tokens
+// uniform and 301 Zipf, E 128 H 2048 I 768: one chain 169 / 190 / 207 / 208 us,
+// 4 up to 32 rows 158 / 175 / 201 / 204, with 2 up to 48 156 / 172 / 197 / 203.
+template <int MODE, bool GATEUP, int MT, int OPEN = 1>
 __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLds<MODE, GATEUP>& s, int e, int m0, int mc,
                                             int ct) {
     using F = Fmt<MODE, GATEUP>;
@@ -182,17 +186,19 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
             for (int q = 0; q < kChunks; ++q) *(v4i*)&s.a[buf][b][aoff + q * kRowStep * 128] = areg[b][q];
     };
     auto load_b = [&](int st, int b, int c) { raw[b][c] = fetch_block<MODE>(rb, wo[c], wo[c] + high, so[c], st * kSub + b); };
-    // kChains: `part` is the running chain and acc the sum of the chains before it
+    // kChains: `part` are the open chains and acc the sum of the chains before them
     constexpr int MP = F::kChains ? MT : 1;
-    typename F::Acc acc[MT][2], part[MP][2];
+    typename F::Acc acc[MT][2], part[OPEN][MP][2];
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi) acc[mi][0] = acc[mi][1] = typename F::Acc{0, 0, 0, 0};
 #pragma unroll
-    for (int mi = 0; mi < MP; ++mi) part[mi][0] = part[mi][1] = typename F::Acc{0, 0, 0, 0};
+    for (int j = 0; j < OPEN; ++j)
+#pragma unroll
+        for (int mi = 0; mi < MP; ++mi) part[j][mi][0] = part[j][mi][1] = typename F::Acc{0, 0, 0, 0};
 
     // Multiply step st; a weight block's registers take the same block of step
     // `next` as soon as it is decoded.
-    auto compute = [&](int st, int next, int buf) {
+    auto compute = [&](int st, int next, int buf, auto open) {
         const int o0 = ((2 * grp) ^ (col % 8)) * 16, o1 = ((2 * grp + 1) ^ (col % 8)) * 16;
 #pragma unroll
         for (int b = 0; b < kSub; ++b) {
@@ -244,7 +250,7 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
                         const v4f rs = *(const v4f*)(GATEUP ? &s.sa[16 * mi + 4 * grp] : &s.rs[GATEUP ? 0 : st * kSub + b][16 * mi + 4 * grp]);
                         v4f d = mfma_fp8(av, lo, zero);
                         if constexpr (MODE == 5) d = mfma_fp8(av, hi, d);
-                        v4f& sum = F::kChains ? part[F::kChains ? mi : 0][c] : acc[mi][c];
+                        v4f& sum = F::kChains ? part[decltype(open)::value][F::kChains ? mi : 0][c] : acc[mi][c];
 #pragma unroll
                         for (int i = 0; i < 4; ++i) sum[i] = fmaf(d[i] * rs[i], sw, sum[i]);
                     }
@@ -278,28 +284,61 @@ __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLd
     // The barrier makes this step's activation rows visible; the buffer staged
     // into was read before it.  The last step loads itself again: no branch
     // around the loads, so the waits stay counted and never drain them.
-    for (int i = 0, st = 0, buf = 0; i < steps; ++i, buf ^= 1) {
-        // kChains: steps w, w + kChains, .. of one chain w after the other
-        const bool end = F::kChains == 0 || st + F::kChains >= steps;
-        const int after = F::kChains == 0 ? st + 1 : end ? st % (F::kChains ? F::kChains : 1) + 1 : st + F::kChains;
-        const int next = i + 1 < steps ? after : st;
-        load_a(next);
-        lds_barrier();
-        compute(st, next, buf);
-        if constexpr (F::kChains > 0) {
-            if (end) {
+    // the chains that end with this step go into the sum
+    auto close_chains = [&] {
 #pragma unroll
-                for (int mi = 0; mi < MT; ++mi) {
+        for (int j = 0; j < OPEN; ++j) {
 #pragma unroll
-                    for (int c = 0; c < 2; ++c) {
-                        acc[mi][c] += part[mi][c];
-                        part[mi][c] = typename F::Acc{0, 0, 0, 0};
-                    }
+            for (int mi = 0; mi < MP; ++mi) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    acc[mi][c] += part[j][mi][c];
+                    part[j][mi][c] = typename F::Acc{0, 0, 0, 0};
                 }
             }
         }
-        stage_a(buf ^ 1);
-        st = next;
+    };
+    constexpr int kC = F::kChains ? F::kChains : 1;
+    if constexpr (OPEN == 1) {
+        for (int i = 0, st = 0, buf = 0; i < steps; ++i, buf ^= 1) {
+            // kChains: blocks w, w + kChains, .. of one chain w after the other
+            const bool end = F::kChains == 0 || st + kC >= steps;
+            const int after = F::kChains == 0 ? st + 1 : end ? st % kC + 1 : st + kC;
+            const int next = i + 1 < steps ? after : st;
+            load_a(next);
+            lds_barrier();
+            compute(st, next, buf, std::integral_constant<int, 0>{});
+            if constexpr (F::kChains > 0) {
+                if (end) close_chains();
+            }
+            stage_a(buf ^ 1);
+            st = next;
+        }
+    } else {
+        // OPEN neighbouring blocks st .., one of each open chain; after the
+        // chains' last ones the next chains open
+        for (int i = 0, st = 0; i < steps; i += OPEN) {
+            const bool end = st + kC >= steps;
+            const int after = end ? st % kC + OPEN : st + kC, last = i + OPEN < steps ? after : st + OPEN - 1;
+            auto step = [&](auto open) {
+                constexpr int J = decltype(open)::value;
+                const int next = J + 1 < OPEN ? st + J + 1 : last;
+                load_a(next);
+                lds_barrier();
+                compute(st + J, next, J % 2, open);
+                if constexpr (J + 1 == OPEN) {
+                    if (end) close_chains();
+                }
+                stage_a(J % 2 ^ 1);
+            };
+            step(std::integral_constant<int, 0>{});
+            step(std::integral_constant<int, 1>{});
+            if constexpr (OPEN == 4) {
+                step(std::integral_constant<int, 2>{});
+                step(std::integral_constant<int, 3>{});
+            }
+            st = after;
+        }
     }
 
     // epilogue: a lane holds column `col` of each 16 x 16 result, rows 4 grp + i
@@ -359,6 +398,14 @@ __global__ __launch_bounds__(kPgThreads, pg_groups(MODE, GATEUP)) void packed_gr
     TileWork t;
     if (!take_tile(a, pg_cols<GATEUP>(a.p.N), t)) return;
     const int e = __builtin_amdgcn_readfirstlane(t.e), m0 = __builtin_amdgcn_readfirstlane(t.m0), mc = t.mc, ct = t.ct;
+    if constexpr (MODE == 5 && GATEUP) {
+        if (a.p.K % 512 == 0 && mc <= 48) {
+            if (mc <= 16) packed_tile<MODE, GATEUP, 1, 4>(a, s, e, m0, mc, ct);
+            else if (mc <= 32) packed_tile<MODE, GATEUP, 2, 4>(a, s, e, m0, mc, ct);
+            else packed_tile<MODE, GATEUP, 3, 2>(a, s, e, m0, mc, ct);
+            return;
+        }
+    }
     if (mc <= 16) packed_tile<MODE, GATEUP, 1>(a, s, e, m0, mc, ct);
     else if (mc <= 32) packed_tile<MODE, GATEUP, 2>(a, s, e, m0, mc, ct);
     else if (mc <= 48) packed_tile<MODE, GATEUP, 3>(a, s, e, m0, mc, ct);

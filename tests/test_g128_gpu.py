@@ -300,7 +300,9 @@ def test_g128_tiled_row_edges(cuda, mode, hidden, inter):
 @pytest.mark.parametrize("mode", [4, 5])
 @pytest.mark.parametrize("hidden,inter,dtype", [
     (256, 512, torch.bfloat16),    # 2 blocks of 128 along K: fewer than the decode kernel's 8 chains
+    (512, 256, torch.bfloat16),    # 4 blocks: chains of one, four of them open
     (1408, 256, torch.float16),    # 11 blocks: chains of two and of one
+    (1536, 256, torch.bfloat16),   # 12 blocks: four open chains of two, four of one
     (2048, 768, torch.bfloat16),   # every chain of two
 ])
 def test_g128_large_calls_give_the_bits_of_small_ones(cuda, mode, hidden, inter, dtype):
@@ -327,7 +329,12 @@ def test_g128_large_calls_give_the_bits_of_small_ones(cuda, mode, hidden, inter,
         assert torch.equal(whole, torch.cat([p[k] for p in parts])), k
     assert torch.equal(backend.forward(x, ids, w, store), out)
 
-    rows, flat, fw = x.repeat_interleave(top_k, 0), ids.reshape(-1, 1), w.reshape(-1, 1).float()
+    # experts of every tile height
+    counts = [1, 16, 17, 32, 33, 0, 48, 49, 64, 65, 0, 3]
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    flat = flat[torch.randperm(len(flat), generator=g)][:, None].to(cuda)
+    rows = torch.randn(len(flat), hidden, generator=g).to(dtype).to(cuda)
+    fw = (torch.rand(len(flat), 1, generator=g) + 0.1).to(cuda)
     pairs = backend.forward_pairs(rows, flat, fw, store)
     split = [backend.forward_pairs(rows[p:p + 64], flat[p:p + 64], fw[p:p + 64], store)
              for p in range(0, len(rows), 64)]
