@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdint>
 #include <map>
 #include <mutex>
@@ -557,12 +558,27 @@ void check_quant_rows(const void* x, int x_dtype, int64_t x_row_stride, int rows
     require(row_div >= 1 && (int64_t)(pairs - 1) / row_div < rows, "pairs read past the activation rows");
 }
 
+// Whether the tiled 8-bit GEMM is the faster one for a projection (modes 1-3).
+// Its tiles run all of K in series, 128 weight rows a workgroup; the
+// column-group kernel's workgroups take 16 rows, split K over 8 waves and walk
+// an expert's pairs in passes of 16.  With few workgroups the chip waits for the
+// tiles' K loops: E 8, N 256, K 4096, 24 pairs INT8 19 us column-group against
+// 33 tiled; E 32, N 1536, K 2048 at 24 / 48 pairs 28 / 35 against 32 / 33; at
+// 1024 pairs 89 against 55.  The line is where a sweep over E 8-128, N 256-4096,
+// K 256-4096 and 8-1024 pairs crosses (at most 28% behind the faster one, 0.2
+// to 0.5% on average); W6A8's decode makes a long K loop dearer.
+bool tiled_projection(const dmoe::QuantProjArgs& q, int experts, int pairs) {
+    if (!dmoe::packed_grouped_fits(q.mode, q.N, q.K, q.w_sn, q.s_sn)) return false;
+    const double active = std::min(pairs, experts), passes = std::max(1.0, pairs / (16 * active));
+    return active * (q.N / 16) * passes * std::sqrt(passes) >= 2048 * (q.mode == 2 ? std::max(1.0, q.K / 3072.0) : 1.0);
+}
+
 // The kernels of a call's grouped projections read the tile map (the tiled
 // ones) or the active-expert list (column-group).
 enum class Grouped { kPacked, kW4A16, kColumns };
 
-Grouped grouped_kind(const dmoe::QuantProjArgs& q) {
-    if (dmoe::packed_grouped_fits(q.mode, q.N, q.K, q.w_sn, q.s_sn)) return Grouped::kPacked;
+Grouped grouped_kind(const dmoe::QuantProjArgs& q, int experts, int pairs) {
+    if (tiled_projection(q, experts, pairs)) return Grouped::kPacked;
     return dmoe::w4a16_grouped_fits(q) ? Grouped::kW4A16 : Grouped::kColumns;
 }
 
@@ -575,7 +591,7 @@ void launch_projection(const dmoe::QuantProjArgs& q, const QuantWorkspace& ws, i
     a.tile_count = ws.tile_count;
     a.max_tiles = std::min(pairs, dmoe::max_block_tiles(pairs, experts, dmoe::kGroupM));
     a.experts = experts;
-    switch (grouped_kind(q)) {
+    switch (grouped_kind(q, experts, pairs)) {
         case Grouped::kPacked: dmoe::launch_packed_grouped(a, stream); break;
         case Grouped::kW4A16: dmoe::launch_w4a16_grouped(a, stream); break;
         default: dmoe::launch_quant_projection(q, std::min(pairs, experts), stream);
@@ -1353,7 +1369,7 @@ int dmoe_quant_projection(const DmoeQuantProj* proj, int experts, int mode, cons
         require(out != nullptr && out_row_stride >= q.N, "output [pairs, N] is required");
         const QuantWorkspace ws = take_quant_workspace(rows, pairs, experts, q.K, 0, workspace, workspace_bytes);
         hipStream_t st = as_stream(stream);
-        const bool tiles = grouped_kind(q) != Grouped::kColumns;
+        const bool tiles = grouped_kind(q, experts, pairs) != Grouped::kColumns;
         quant_group(ids, ids_dtype, pairs, experts, ws, tiles, !tiles, status, st);
         quant_operand(q, x, x_dtype, x_row_stride, rows, q.K, ws.xq, ws.xs, st);
         q.row_div = row_div;
@@ -1426,8 +1442,8 @@ static void quant_forward_impl(const DmoeQuantBank* bank, const void* x, int x_d
         }
         up.gateup = 1;
         const auto grouped = [&](bool tiled) {
-            return (!small_up && (grouped_kind(up) != Grouped::kColumns) == tiled) ||
-                   (!small_dn && (grouped_kind(dn) != Grouped::kColumns) == tiled);
+            return (!small_up && (grouped_kind(up, E, pairs) != Grouped::kColumns) == tiled) ||
+                   (!small_dn && (grouped_kind(dn, E, pairs) != Grouped::kColumns) == tiled);
         };
         if (!small_up || !small_dn) quant_group(ids, ids_dtype, pairs, E, ws, grouped(true), grouped(false), status, st);
 
