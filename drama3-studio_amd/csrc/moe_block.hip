@@ -19,7 +19,7 @@
 // wave reads the same few kilobytes, so they stay in L2) with the row's own
 // loads: one memory round trip at batch 1.  Sums are wave-wide by DPP.
 //
-// Calls of more than kBlkGemvTokens tokens take the tiled form of the same two
+// Calls of many tokens (block_tiled) take the tiled form of the same two
 // launches (block_gemm_*_kernel below): the work is then a small dense GEMM
 // and the GEMV's fp32 multiply-adds bound it.
 #include <algorithm>
@@ -33,9 +33,7 @@ namespace {
 
 constexpr int kBlkWaves = 4, kBlkThreads = kBlkWaves * kWave;
 constexpr int kBlkTokens = 2;           // token rows held in registers per chunk
-// Calls of more tokens take the tiled kernels: pre + post at hidden 2048, 128
-// experts, inter 768 measured 20.7 (GEMV) vs 23.2 us (tiled) at 9 tokens, 25.4
-// vs 23.2 at 12, 112 vs 26.7 at 64 and 864 vs 32.0 at 509.
+// Calls of at most this many tokens take the GEMV (block_tiled).
 constexpr int kBlkGemvTokens = 10;
 constexpr int kBlkMaxK = 4096;          // reduction length (hidden or shared intermediate)
 
@@ -173,8 +171,9 @@ __global__ __launch_bounds__(kBlkThreads) void block_post_kernel(BlockPostArgs a
 // each, K in steps of 128 columns double-buffered in LDS through registers:
 // step s + 1 is in flight while step s is multiplied, one barrier per step;
 // two workgroups per CU (64 KB of LDS each) cover each other's waits.  The
-// serial chain of 16 + 6 steps bounds these shapes (3.5 GFLOP over 9 MB at 509
-// tokens: 20 us pre, 12 us post); four steps in flight measured no better.
+// serial chain of 16 + 6 steps bounds these shapes (509 tokens: pre 3.5 GFLOP
+// over 10 MB in 20 us, post 1.6 GFLOP over 10 MB in 12; 18 and 12 at 64);
+// four steps in flight measured no better.
 // The 16-byte chunk c of tile row r sits at chunk c ^ (r % 16), so the 16 rows
 // of an operand read touch all banks.  Columns past K and rows past the
 // matrices are zero.
@@ -328,12 +327,23 @@ bool block_fits(int hidden, int shared_inter) {
            shared_inter % 8 == 0;
 }
 
-// The tiled kernels take every call past the GEMV's range that a grid's y
-// dimension can cover.
-static bool block_tiled(int tokens) { return tokens > kBlkGemvTokens && tokens <= 65535 * kBgTile; }
+// The GEMV's time grows with its tokens and, once its rows fill the chip, with
+// the rows; the tiled kernel's with its 128-column steps, which run in series.
+// `tokens` x `rows` (at least `fill`, the rows that cost no more than fewer) is
+// held against their crossing, (per_step * steps + base) / 10 tokens.  Measured,
+// GEMV / tiled: pre at hidden 2048, 1665 rows 13.9 / 16.5 us at 11 tokens, 16.9
+// / 16.8 at 14, 61 / 18 at 64; at 4096, 3329 rows 27.6 / 28.9 at 12, 34.7 / 28.8
+// at 16; at 256, 145 rows 14.0 / 6.5 at 11.  Post at inter 2048, 512 rows 16.6 /
+// 18.5 at 20, 19.1 / 18.6 at 24; at 768, 2048 rows 12.4 / 9.4 at 11.  The tiled
+// grid's y dimension bounds it above.
+static bool block_tiled(int tokens, int rows, int fill, int k, int per_step, int base) {
+    const int64_t steps = (k + kBgK - 1) / kBgK;
+    return tokens > kBlkGemvTokens && tokens <= 65535 * kBgTile &&
+           (int64_t)tokens * std::max(rows, fill) * 10 > (per_step * steps + base) * fill;
+}
 
 void launch_block_pre(const BlockPreArgs& a, int cus, hipStream_t stream) {
-    if (block_tiled(a.tokens)) {
+    if (block_tiled(a.tokens, a.experts + 1 + 2 * a.shared_inter, 1664, a.hidden, 8, 13)) {
         const dim3 tiles(block_router_tiles(a.experts) + (a.shared_inter + kBgActCols - 1) / kBgActCols,
                          (a.tokens + kBgTile - 1) / kBgTile);
         hipLaunchKernelGGL(block_gemm_pre_kernel, tiles, dim3(kBlkThreads), 0, stream, a);
@@ -345,7 +355,7 @@ void launch_block_pre(const BlockPreArgs& a, int cus, hipStream_t stream) {
 }
 
 void launch_block_post(const BlockPostArgs& a, int cus, hipStream_t stream) {
-    if (block_tiled(a.tokens)) {
+    if (block_tiled(a.tokens, a.hidden, 2048, a.shared_inter, 12, 38)) {
         const dim3 tiles((a.hidden + kBgTile - 1) / kBgTile, (a.tokens + kBgTile - 1) / kBgTile);
         hipLaunchKernelGGL(block_gemm_post_kernel, tiles, dim3(kBlkThreads), 0, stream, a);
         return;

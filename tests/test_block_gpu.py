@@ -65,6 +65,9 @@ def test_block_pre_and_post_match_oracle(cuda, tokens):
     (64, 136, 64, 40),     # one full row tile; the shared gate alone in a tile; K and inter past a step / tile
     (65, 1032, 13, 104),   # one row in the second row tile
     (130, 264, 5, 8),      # the smallest inter
+    (14, 2048, 16, 64),    # before the crossing of a deep K: GEMV logits, tiled post
+    (15, 2048, 16, 64),    # past it
+    (22, 512, 8, 2048),    # the other way round: tiled logits, GEMV post
 ])
 def test_block_tiled_calls_match_oracle(cuda, tokens, hidden, experts, inter):
     """Tile edges of the many-token kernels, with padded row strides."""
