@@ -416,7 +416,7 @@ __global__ __launch_bounds__(kPgThreads, pg_groups(MODE, GATEUP)) void packed_gr
 
 // Whole K steps, and an expert's rows within 32-bit byte offsets.
 bool packed_grouped_fits(int mode, int N, int K, int64_t w_sn, int64_t s_sn) {
-    return mode >= 1 && mode <= 5 && K % (mode == 1 ? 128 : 256) == 0 && N * w_sn < (int64_t(1) << 32) &&
+    return mode >= 1 && mode <= 5 && K % (128 * std::max(pg_sub(mode, true), pg_sub(mode, false))) == 0 && N * w_sn < (int64_t(1) << 32) &&
            N * s_sn < (int64_t(1) << 32);
 }
 

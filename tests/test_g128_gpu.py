@@ -2,8 +2,9 @@
 W6A8-g128 (mode 5): 4- / 6-bit codes with one fp16 scale per (row,
 128-group), FP8 per-token activations -- against the oracle.
 
-They run on the FP8 decode kernels with the integer levels expanded into
-E4M3 MFMA operands in registers.  Bars: routing ids bit-exact; outputs within
+Calls of up to 256 pairs run on the FP8 decode kernels, larger ones on the
+tiled GEMMs with the same sums, with the integer levels expanded into E4M3 MFMA
+operands in registers.  Bars: routing ids bit-exact; outputs within
 ||y - r||_inf / ||r||_inf <= 2e-2 of the oracle; the single-launch and the
 three-launch decode bit-identical; hipGraph replays identical to eager calls.
 """
@@ -93,8 +94,8 @@ def test_g128_layer_matches_oracle_and_both_decodes_agree(cuda, decode_mode, mod
 
 @pytest.mark.parametrize("mode", [4, 5])
 def test_g128_pairs_beyond_one_decode_call_and_invalid_ids(cuda, mode):
-    """600 single-pair rows run as three consecutive decode calls; rows with
-    ids outside [0, E) are zero and flag the status word."""
+    """600 single-pair rows, more than a decode call holds; rows with ids
+    outside [0, E) are zero and flag the status word."""
     print_case("g128 pairs", mode)
     store = bank_on(cuda, mode, 16, 512, 256, 77 + mode)
     g = torch.Generator().manual_seed(5 + mode)
@@ -118,7 +119,8 @@ def test_g128_pairs_beyond_one_decode_call_and_invalid_ids(cuda, mode):
 
 @pytest.mark.parametrize("mode", [4, 5])
 def test_g128_prefill_tokens_as_consecutive_decode_calls(cuda, mode):
-    """A 100-token layer call (800 pairs) against the oracle on spread tokens."""
+    """A 100-token layer call (800 pairs: tiled GEMMs; consecutive decode calls
+    only where the workspace holds no more) against the oracle on spread tokens."""
     print_case("g128 prefill", mode)
     store = bank_on(cuda, mode, 32, 1024, 256, 31 + mode)
     g = torch.Generator().manual_seed(99)
@@ -126,7 +128,7 @@ def test_g128_prefill_tokens_as_consecutive_decode_calls(cuda, mode):
     ids, w = orc.route_topk(torch.randn(100, 32, generator=g).numpy(), 8)
     weights = torch.from_numpy(w).bfloat16()
     out = QuantizedExpertBackend(mode).forward(x.to(cuda), torch.from_numpy(ids).to(cuda), weights.to(cuda), store)
-    pick = [0, 31, 32, 63, 64, 99]  # both sides of every 32-token chunk boundary
+    pick = [0, 31, 32, 63, 64, 99]  # both sides of what would be decode calls
     expected = oracle_layer(store, x.float().numpy()[pick], ids[pick], weights.float().numpy()[pick])
     assert rel_inf(out.float().cpu().numpy()[pick], expected) < TOL
 
@@ -171,9 +173,8 @@ def test_g128_24_layer_decode_step_in_hipgraph(cuda, mode):
 @pytest.mark.parametrize("mode", [4, 5])
 def test_g128_routed_layer_above_one_decode_call(cuda, mode):
     """Router + experts of a 100-token call (800 pairs): the router kernel
-    writes the routing, the experts run as consecutive decode calls over it.
-    Routing bit-exact with the oracle on every token, outputs within 2e-2 of
-    the oracle on tokens at both sides of every decode-call boundary."""
+    writes the routing, the tiled GEMMs run over it.  Routing bit-exact with the
+    oracle on every token, outputs within 2e-2 of the oracle on spread tokens."""
     print_case("g128 routed 100 tokens", mode)
     store = bank_on(cuda, mode, 32, 1024, 256, 51 + mode)
     g = torch.Generator().manual_seed(700 + mode)
@@ -234,8 +235,9 @@ def test_g128_moe_block_prefill_size(cuda, mode):
 @pytest.mark.parametrize("mode", [4, 5])
 def test_g128_layer_combine_with_pairs_per_row_not_top_k(cuda, mode):
     """A direct C-ABI layer call whose rows hold 2 pairs each while tokens
-    hold 3 (row_div 2, top_k 3, 600 pairs): decode calls cut at whole tokens
-    and rows, so every token equals the oracle's sum of its three pairs."""
+    hold 3 (row_div 2, top_k 3, 600 pairs): every token equals the oracle's sum
+    of its three pairs, by the tiled GEMMs and, with a workspace that holds
+    decode calls only, by decode calls cut at whole tokens and rows, alike."""
     import ctypes
 
     from drama_moe.offload import device_state
@@ -249,18 +251,21 @@ def test_g128_layer_combine_with_pairs_per_row_not_top_k(cuda, mode):
     x = torch.randn(rows, 512, generator=g).bfloat16()
     ids = torch.randint(0, 16, (pairs,), generator=g)
     w = (torch.rand(pairs, generator=g) + 0.1).float()
-    out = torch.empty(tokens, 512, dtype=torch.float32, device=cuda)
+    outs = torch.empty(2, tokens, 512, dtype=torch.float32, device=cuda)
     xd, idd, wd = x.to(cuda), ids.to(cuda), w.to(cuda)
     lib = _lib.library()
     bank = bank_struct(store)
     state = device_state(cuda)
     ws = state.workspace_for(lib.dmoe_quant_workspace_bytes(ctypes.byref(bank), rows, pairs))
-    _lib.check(lib.dmoe_quant_moe_forward(
-        ctypes.byref(bank), _lib.ptr(xd), _lib.dtype_code(xd.dtype), xd.stride(0), rows, row_div, _lib.ptr(idd),
-        _lib.dtype_code(idd.dtype), _lib.ptr(wd), _lib.dtype_code(wd.dtype), pairs, top_k, _lib.ptr(out),
-        _lib.F32, out.stride(0), None, _lib.ptr(ws), ws.numel(), _lib.ptr(state.status),
-        _lib.stream_handle(cuda)))
+    for out, room in zip(outs, (ws.numel(), lib.dmoe_quant_workspace_bytes(ctypes.byref(bank), 256, 256))):
+        _lib.check(lib.dmoe_quant_moe_forward(
+            ctypes.byref(bank), _lib.ptr(xd), _lib.dtype_code(xd.dtype), xd.stride(0), rows, row_div, _lib.ptr(idd),
+            _lib.dtype_code(idd.dtype), _lib.ptr(wd), _lib.dtype_code(wd.dtype), pairs, top_k, _lib.ptr(out),
+            _lib.F32, out.stride(0), None, _lib.ptr(ws), room, _lib.ptr(state.status),
+            _lib.stream_handle(cuda)))
     torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    out = outs[0]
     b13, b2 = oracle_banks(store)
     xs = x.float().numpy()
     parts = np.concatenate([orc.fp8_expert_pairs(b13, b2, xs[p // row_div], ids[p:p + 1].numpy(),
@@ -274,8 +279,7 @@ def test_g128_layer_combine_with_pairs_per_row_not_top_k(cuda, mode):
 def test_g128_tiled_row_edges(cuda, mode, hidden, inter):
     """More pairs than one decode call: the tiled GEMMs with experts of 1, 16,
     17, 32, 33, 48, 49, 64, 65 and 0 rows, invalid ids and an intermediate size
-    above and below the hidden one; inter 384 is no whole K step and runs as
-    consecutive decode calls."""
+    above and below the hidden one, 384 an odd number of K blocks."""
     print_case("g128 tiled edges", mode, hidden, inter)
     counts = [1, 16, 17, 32, 33, 0, 48, 49, 64, 65]
     store = bank_on(cuda, mode, len(counts), hidden, inter, 11 + mode)
