@@ -135,7 +135,8 @@ __device__ __forceinline__ BlockRaw<MODE> fetch_block(const RowBase& rb, uint32_
 // visit neighbouring blocks; the registers hold 4 chains up to 32 rows, 2 up to
 // 48 and one above (2 above: 51 spills).  A layer at 40 / 128 / 600 tokens
 // uniform and 301 Zipf, E 128 H 2048 I 768: one chain 169 / 190 / 207 / 208 us,
-// 4 up to 32 rows 158 / 175 / 201 / 204, with 2 up to 48 156 / 172 / 197 / 203.
+// 4 up to 32 rows 158 / 175 / 201 / 204, with 2 up to 48 156 / 172 / 197 / 203
+// (W4A8-g128, one plane: 112 / 130 / 148 / 151 -> 111 / 129 / 145 / 150).
 template <int MODE, bool GATEUP, int MT, int OPEN = 1>
 __device__ __forceinline__ void packed_tile(const PackedGroupedArgs& a, PackedLds<MODE, GATEUP>& s, int e, int m0, int mc,
                                             int ct) {
@@ -398,7 +399,7 @@ __global__ __launch_bounds__(kPgThreads, pg_groups(MODE, GATEUP)) void packed_gr
     TileWork t;
     if (!take_tile(a, pg_cols<GATEUP>(a.p.N), t)) return;
     const int e = __builtin_amdgcn_readfirstlane(t.e), m0 = __builtin_amdgcn_readfirstlane(t.m0), mc = t.mc, ct = t.ct;
-    if constexpr (MODE == 5 && GATEUP) {
+    if constexpr (Fmt<MODE, GATEUP>::kChains > 0) {
         if (a.p.K % 512 == 0 && mc <= 48) {
             if (mc <= 16) packed_tile<MODE, GATEUP, 1, 4>(a, s, e, m0, mc, ct);
             else if (mc <= 32) packed_tile<MODE, GATEUP, 2, 4>(a, s, e, m0, mc, ct);
