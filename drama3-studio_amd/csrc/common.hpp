@@ -60,6 +60,8 @@ __device__ __forceinline__ float load_as_f32(const void* p, int64_t i, int dtype
     return ((const float*)p)[i];
 }
 
+__device__ __forceinline__ float bf16_round(float v) { return (float)(__bf16)v; }
+
 __device__ __forceinline__ void store_from_f32(void* p, int64_t i, int dtype, float v) {
     if (dtype == kBF16) ((uint16_t*)p)[i] = f32_to_bf16(v);
     else if (dtype == kF16) ((uint16_t*)p)[i] = f32_to_f16(v);

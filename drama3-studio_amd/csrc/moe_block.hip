@@ -39,7 +39,6 @@ constexpr int kBlkMaxK = 4096;          // reduction length (hidden or shared in
 
 __device__ __forceinline__ float bf16v(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ uint16_t to_bf16(float v) { return __builtin_bit_cast(uint16_t, (__bf16)v); }
-__device__ __forceinline__ float bf16r(float v) { return (float)(__bf16)v; }
 
 // dot of this lane's 8-element slices (bf16 pairs in v4i) accumulated into acc.
 __device__ __forceinline__ float dot8(const v4i& w, const v4i& x, float acc) {
@@ -118,12 +117,12 @@ __global__ __launch_bounds__(kBlkThreads) void block_pre_kernel(BlockPreArgs a) 
                 // every lane holds every sum; lane t writes token t
 #pragma unroll
                 for (int t = 0; t < kBlkTokens; ++t)
-                    if (lane == t && t < n) a.logits[(int64_t)(t0 + t) * a.logits_row_stride + r] = bf16r(y[t]);
+                    if (lane == t && t < n) a.logits[(int64_t)(t0 + t) * a.logits_row_stride + r] = bf16_round(y[t]);
             } else if (r == E) {
 #pragma unroll
                 for (int t = 0; t < kBlkTokens; ++t)
                     if (lane == t && t < n) {
-                        const float g = bf16r(y[t]);
+                        const float g = bf16_round(y[t]);
                         a.sgate[t0 + t] = to_bf16(1.0f / (1.0f + expf(-g)));
                     }
             } else {
@@ -132,8 +131,8 @@ __global__ __launch_bounds__(kBlkThreads) void block_pre_kernel(BlockPreArgs a) 
 #pragma unroll
                 for (int t = 0; t < kBlkTokens; ++t)
                     if (lane == t && t < n) {
-                        const float g = bf16r(y[t]), up = bf16r(u[t]);
-                        const float sg = bf16r(g / (1.0f + expf(-g)));
+                        const float g = bf16_round(y[t]), up = bf16_round(u[t]);
+                        const float sg = bf16_round(g / (1.0f + expf(-g)));
                         a.act[(int64_t)(t0 + t) * a.act_row_stride + j] = to_bf16(sg * up);
                     }
             }
@@ -157,9 +156,9 @@ __global__ __launch_bounds__(kBlkThreads) void block_post_kernel(BlockPostArgs a
             for (int t = 0; t < kBlkTokens; ++t)
                 if (lane == t && t < n) {
                     const int64_t tt = t0 + t;
-                    const float s = bf16r(bf16v(a.sgate[tt]) * bf16r(y[t]));
+                    const float s = bf16_round(bf16v(a.sgate[tt]) * bf16_round(y[t]));
                     const float e = bf16v(a.experts[tt * a.experts_row_stride + r]);
-                    const float m = bf16r(e + s);
+                    const float m = bf16_round(e + s);
                     a.out[tt * a.out_row_stride + r] = to_bf16(bf16v(a.residual[tt * a.residual_row_stride + r]) + m);
                 }
         }
@@ -279,14 +278,14 @@ __global__ __launch_bounds__(kBlkThreads, 2) void block_gemm_pre_kernel(BlockPre
 #pragma unroll
                 for (int ni = 0; ni < 2; ++ni) {
                     const int n = n0 + 32 * (wave % 2) + 16 * ni + col;
-                    const float y = bf16r(acc[mi][ni][i]);
+                    const float y = bf16_round(acc[mi][ni][i]);
                     if (n < E) a.logits[t * a.logits_row_stride + n] = y;
                     else if (n == E) a.sgate[t] = to_bf16(1.0f / (1.0f + expf(-y)));
                 }
             } else {
                 const int j = n0 + 16 * (wave % 2) + col;
-                const float g = bf16r(acc[mi][0][i]), up = bf16r(acc[mi][1][i]);
-                if (j < I) a.act[t * a.act_row_stride + j] = to_bf16(bf16r(g / (1.0f + expf(-g))) * up);
+                const float g = bf16_round(acc[mi][0][i]), up = bf16_round(acc[mi][1][i]);
+                if (j < I) a.act[t * a.act_row_stride + j] = to_bf16(bf16_round(g / (1.0f + expf(-g))) * up);
             }
         }
     }
@@ -312,8 +311,8 @@ __global__ __launch_bounds__(kBlkThreads, 2) void block_gemm_post_kernel(BlockPo
             for (int ni = 0; ni < 2; ++ni) {
                 const int n = n0 + 32 * (wave % 2) + 16 * ni + col;
                 if (n >= H) continue;
-                const float sh = bf16r(sg * bf16r(acc[mi][ni][i]));
-                const float m = bf16r(bf16v(a.experts[t * a.experts_row_stride + n]) + sh);
+                const float sh = bf16_round(sg * bf16_round(acc[mi][ni][i]));
+                const float m = bf16_round(bf16v(a.experts[t * a.experts_row_stride + n]) + sh);
                 a.out[t * a.out_row_stride + n] = to_bf16(bf16v(a.residual[t * a.residual_row_stride + n]) + m);
             }
         }

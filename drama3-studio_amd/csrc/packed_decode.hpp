@@ -17,8 +17,6 @@ __device__ __forceinline__ uint32_t pack_f16(float a, float b) {
     return (uint32_t)f32_to_f16(a) | ((uint32_t)f32_to_f16(b) << 16);
 }
 
-__device__ __forceinline__ float bf16_round(float v) { return (float)(__bf16)v; }
-
 // E4M3 byte -> fp32 (hardware decode of one byte).
 __device__ __forceinline__ float e4m3(uint32_t byte) { return fp8x2_to_f32(byte & 0xFFu, false)[0]; }
 

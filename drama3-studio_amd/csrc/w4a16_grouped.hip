@@ -39,6 +39,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "packed_decode.hpp"
 #include "tile_map.hpp"
 
 namespace dmoe {
@@ -59,18 +60,6 @@ struct alignas(16) W4Lds {
     int pair[kW4Rows];            // original pair of each chunk row (-1: past the expert)
 };
 
-// Zero-point word of banks without qzeros: zero point 8 in every nibble.
-__device__ int32_t g_w4_zero8 = (int32_t)0x88888888u;
-
-__device__ __forceinline__ uint32_t pack2(float a, float b, bool f16) {
-    if (f16) return (uint32_t)f32_to_f16(a) | ((uint32_t)f32_to_f16(b) << 16);
-    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-    const v2bf p = {(__bf16)a, (__bf16)b};
-    return __builtin_bit_cast(uint32_t, p);
-}
-
-__device__ __forceinline__ float bf16r(float v) { return (float)(__bf16)v; }
-
 // The raw weight bytes of one lane for one column tile and K block.
 struct W4Raw {
     v4i codes;       // 32 nibbles: word t = K [32 g + 8 t, +8), nibble i = + i
@@ -83,7 +72,7 @@ __device__ __forceinline__ W4Raw w4_fetch(const QuantProjArgs& a, const uint8_t*
     W4Raw r;
     r.codes = *(const v4i*)(wrow + kb * 64 + g * 16);
     r.scale = *(const uint16_t*)(srow + kb * 2);
-    r.zeros = (uint32_t)*(a.z ? zrow + (int64_t)kb * (a.N / 8) : &g_w4_zero8);
+    r.zeros = (uint32_t)*(a.z ? zrow + (int64_t)kb * (a.N / 8) : &g_zero_point8);
     return r;
 }
 
@@ -117,7 +106,7 @@ __device__ __forceinline__ void w4_dequant(const W4Raw& r, int n, v4i (&op)[4]) 
                             fmaf((float)c04[1], s1, b1), fmaf((float)c15[1], s16, b16),
                             fmaf((float)c26[1], s1, b1), fmaf((float)c37[1], s16, b16)};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) op[t][i] = (int)pack2(v[2 * i], v[2 * i + 1], F16);
+        for (int i = 0; i < 4; ++i) op[t][i] = (int)(F16 ? pack_f16(v[2 * i], v[2 * i + 1]) : pack_bf16(v[2 * i], v[2 * i + 1]));
     }
 }
 
@@ -247,13 +236,13 @@ __global__ __launch_bounds__(kW4Threads) void w4a16_grouped_kernel(PackedGrouped
                 const int p = s.pair[16 * mi + 4 * g + i];
                 if (p < 0) continue;
                 if constexpr (GATEUP) {
-                    const float yg = bf16r(acc[mi][0][i]), yu = bf16r(acc[mi][1][i]);
-                    const float act = bf16r(bf16r(yg / (1.0f + expf(-yg))) * yu);
+                    const float yg = bf16_round(acc[mi][0][i]), yu = bf16_round(acc[mi][1][i]);
+                    const float act = bf16_round(bf16_round(yg / (1.0f + expf(-yg))) * yu);
                     a.act[(int64_t)p * half + n[0]] = __builtin_bit_cast(uint16_t, (__bf16)act);
                 } else {
 #pragma unroll
                     for (int c = 0; c < 2; ++c) {
-                        const float y = bf16r(acc[mi][c][i]);
+                        const float y = bf16_round(acc[mi][c][i]);
                         if (a.weighted)
                             ((float*)a.out)[(int64_t)p * a.out_row_stride + n[c]] = y * load_as_f32(a.weights, p, a.w_dtype);
                         else
