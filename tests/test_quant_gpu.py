@@ -421,8 +421,11 @@ def test_tiled_projection_row_and_column_edges(cuda, mode, n, k, weighted):
     ids = flat[torch.randperm(len(flat), generator=g)]
     x = torch.randn(len(ids), k, generator=g).bfloat16()
     w = torch.rand(len(ids), generator=g) + 0.1
+    backend = quantized.QuantizedExpertBackend(mode)
+    backend.status(cuda)
     out = quantized.projection(x.to(cuda), ids.to(cuda), w.to(cuda), bank.to(cuda), scales.to(cuda), mode=mode,
                                weighted=weighted)
+    assert backend.status(cuda) == _lib.STATUS_BAD_EXPERT_ID  # and cleared for the tests after this one
     keep = [r for r in range(len(ids)) if 0 <= int(ids[r]) < len(counts)]
     assert torch.bincount(ids[keep], minlength=len(counts)).tolist() == counts
     b = orc.QuantBank(mode, bank.contiguous().numpy(), scales.contiguous().numpy(), n, k)
