@@ -628,9 +628,10 @@ void quant_operand(dmoe::QuantProjArgs& q, const void* x, int x_dtype, int64_t x
 }
 
 // ------------------------------------------- group-128 integer banks (4, 5)
-// W4A8-g128 / W6A8-g128 packed banks run on the FP8 decode kernels: their
-// integer levels expand exactly into E4M3 MFMA operands (wfmt.hpp), with the
-// activations quantized to FP8 per token.
+// W4A8-g128 / W6A8-g128 packed banks run on the FP8 decode kernels, calls above
+// 256 pairs on the tiled GEMMs of packed_grouped.hip: their integer levels
+// expand exactly into E4M3 MFMA operands (wfmt.hpp), with the activations
+// quantized to FP8 per token.
 
 bool is_g128_mode(int mode) { return mode == 4 || mode == 5; }
 

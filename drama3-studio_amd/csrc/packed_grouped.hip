@@ -26,11 +26,12 @@
 // the expert's last pair are skipped in 16-row units (1 to 4 of them).
 // Modes 4-5 store the hidden fp32; one pass quantizes it for the down kernel.
 //
-// Measured (first form) gate/up + down against the column-group kernel (modes 1-3: 16
-// columns a workgroup, 16 rows a pass) and consecutive decode calls (4-5):
-// INT8 197 tokens 276 + 313 -> 90 + 61 us (4.1 TB/s of weights), W6A8 512
-// tokens 201 + 194 -> 112 + 69 us, W6A8-g128 301 tokens 2383 (layer) -> 120 +
-// 64 us.  Decode VALU and its latency bound the 6-bit formats.
+// Measured gate/up + down against the column-group kernel (modes 1-3: 16 columns
+// a workgroup, 16 rows a pass) and consecutive decode calls (4-5), E 128 H 2048
+// I 768: INT8 197 tokens 276 + 313 -> 87 + 57 us (4.2 TB/s), W6A8 512 tokens 201
+// + 194 -> 117 + 72 us, a W6A8-g128 layer at 301 tokens 2419 -> 201 us.  INT8
+// waits for its one K step of loads; decode instructions and their latency bound
+// the 6-bit formats.  (Small banks: see tiled_projection in abi.cpp.)
 #include <algorithm>
 #include <type_traits>
 

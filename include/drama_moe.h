@@ -329,8 +329,10 @@ DMOE_API int dmoe_fp8_moe_layer_noalloc(const DmoeFp8Bank* bank, const void* x, 
  * quantized to FP8 per token (scale = max(amax, 1e-10) * fl(1/448) over the
  * row), with the FP8 W8A8 contract otherwise (block fma chain, gate/up
  * rounded through the activation dtype, FP8 128-group hidden, slot-order
- * combine); they run on the FP8 decode kernels, calls above 256 route pairs
- * as consecutive decode calls.
+ * combine).  Calls of up to 256 route pairs run on the FP8 decode kernels,
+ * larger ones as tiled grouped GEMMs, or, where the workspace holds no more
+ * than a call of 256 pairs needs, as consecutive decode calls: the same bits
+ * every way, so a row's result does not depend on how its call is split.
  * Strides are in bytes (zeros: int32 elements per expert).  K is a multiple
  * of 128 (modes 0, 4, 5) or 256 (modes 1-3), at most 4096 (modes 0-3) or
  * 8192 (modes 4, 5); N a multiple of 16. */
@@ -359,7 +361,10 @@ DMOE_API int dmoe_rotate_quantize(const void* x, int x_dtype, int64_t x_row_stri
                                   int8_t* q, float* scales, void* stream);
 
 /* Workspace bytes of a packed-bank call over `rows` activation rows and
- * `pairs` route pairs (zero-filled once, reused; see dmoe_fp8_workspace_bytes). */
+ * `pairs` route pairs (zero-filled once, reused; see dmoe_fp8_workspace_bytes).
+ * Modes 4 and 5 above 256 pairs: H * 5 + I bytes a pair and their scales (H
+ * >= I; 11 KB at H 2048, I 768); with the bytes for 256 pairs instead such a
+ * call runs as consecutive decode calls. */
 DMOE_API size_t dmoe_quant_workspace_bytes(const DmoeQuantBank* bank, int rows, int pairs);
 
 /* Workspace bytes of dmoe_quant_projection over `rows` activation rows of K
@@ -433,7 +438,9 @@ DMOE_API int dmoe_w4a16_linear(const void* x, int x_dtype, int64_t x_row_stride,
  * input of dmoe_*_moe_layer --, shared_gate_out [tokens] bf16 =
  * bf16(sigmoid(bf16(x shared_gate_w^T))) (shared_gate_w: the [1, hidden]
  * shared_expert_gate weight) and shared_act [tokens, shared_inter] bf16 =
- * bf16(bf16(silu(bf16(x gate_proj^T))) * bf16(x up_proj^T)). */
+ * bf16(bf16(silu(bf16(x gate_proj^T))) * bf16(x up_proj^T)).  The sums are
+ * fp32, in one order for few tokens and another for many (more than 10, by
+ * shape): the same row's bf16 logit may differ by one step between the two. */
 DMOE_API int dmoe_moe_block_pre(const void* x, int64_t x_row_stride, int tokens, int hidden,
                                 const void* router_w, int64_t router_row_stride, int experts,
                                 const void* shared_gate_w, const void* gate_proj, int64_t gate_row_stride,
