@@ -308,6 +308,8 @@ def test_g128_tiled_row_edges(cuda, mode, hidden, inter):
     (1408, 256, torch.float16),    # 11 blocks: chains of two and of one
     (1536, 256, torch.bfloat16),   # 12 blocks: four open chains of two, four of one
     (2048, 768, torch.bfloat16),   # every chain of two
+    (4096, 128, torch.bfloat16),   # chains of four, open side by side
+    (4224, 128, torch.float16),    # 33 blocks: chains of five and four, one at a time
 ])
 def test_g128_large_calls_give_the_bits_of_small_ones(cuda, mode, hidden, inter, dtype):
     """A route row's value does not depend on how its call is split: calls of
